@@ -25,11 +25,13 @@ namespace {
 // Copies run on the context's stream and are waited for (the source is a
 // temporary): the legacy null stream would wait for every other context's
 // stream in the process and break another thread's graph capture.
+// pad: spare entries behind the array, zero.
 template <typename X>
-X *dev_upload(hipStream_t s, const std::vector<X> &h) {
+X *dev_upload(hipStream_t s, const std::vector<X> &h, size_t pad = 0) {
     X *p = nullptr;
-    size_t bytes = sizeof(X) * std::max<size_t>(h.size(), 1);
+    size_t bytes = sizeof(X) * std::max<size_t>(h.size() + pad, 1);
     JDHIP_CHECK(hipMalloc(&p, bytes));
+    if (pad) JDHIP_CHECK(hipMemsetAsync(p + h.size(), 0, sizeof(X) * pad, s));
     if (!h.empty()) {
         JDHIP_CHECK(hipMemcpyAsync(p, h.data(), sizeof(X) * h.size(), hipMemcpyHostToDevice, s));
         JDHIP_CHECK(hipStreamSynchronize(s));
@@ -233,8 +235,7 @@ struct DevLevel {
     int *lct_ptr = nullptr, *lct_idx = nullptr;
     T *lct_val = nullptr;
     // row blocks of the CSR-stream form for L_B, L_B^T, L_CB, L_CB^T
-    int *rb_b = nullptr, *rb_t = nullptr, *rb_c = nullptr, *rb_ct = nullptr;
-    int nrb_b = 0, nrb_t = 0, nrb_c = 0, nrb_ct = 0;
+    StreamView st_b, st_t, st_c, st_ct;
     std::vector<int> fwd_ptr, bwd_ptr;  // host level pointers
     int *fwd_rows = nullptr, *bwd_rows = nullptr;
     W *buf = nullptr, *out = nullptr, *t1 = nullptr, *t2 = nullptr;  // work vectors
@@ -355,16 +356,16 @@ class IldlImpl : public IldlImplBase {
             sort_rows(nB, bp, bi, bv);
             sort_rows(nC, cp, ci, cv);
             D.lb_ptr = track(dev_upload(ctx_->stream, bp));
-            D.lb_idx = track(dev_upload(ctx_->stream, bi));
-            D.lb_val = track(dev_upload(ctx_->stream, bv));
+            D.lb_idx = track(dev_upload(ctx_->stream, bi, kStreamPad));
+            D.lb_val = track(dev_upload(ctx_->stream, bv, kStreamPad));
             std::vector<int> tp, ti;
             std::vector<T> tv;
             transpose(nB, nB, bp, bi, bv, tp, ti, tv);
             D.lt_ptr = track(dev_upload(ctx_->stream, tp));
-            D.lt_idx = track(dev_upload(ctx_->stream, ti));
-            D.lt_val = track(dev_upload(ctx_->stream, tv));
-            upload_row_blocks(nB, bp, D.rb_b, D.nrb_b);
-            upload_row_blocks(nB, tp, D.rb_t, D.nrb_t);
+            D.lt_idx = track(dev_upload(ctx_->stream, ti, kStreamPad));
+            D.lt_val = track(dev_upload(ctx_->stream, tv, kStreamPad));
+            D.st_b = upload_stream(nB, bp, bi);
+            D.st_t = upload_stream(nB, tp, ti);
             D.sf = upload_sell(build_sell(nB, bp, bi, bv, sigma_));
             D.sb = upload_sell(build_sell(nB, tp, ti, tv, sigma_));
             // dependency levels from the triangular (factor) numbering
@@ -381,17 +382,17 @@ class IldlImpl : public IldlImplBase {
             }
             D.sc = upload_sell(build_sell(nC, cp, ci, cv, sigma_, true));
             D.lc_ptr = track(dev_upload(ctx_->stream, cp));
-            D.lc_idx = track(dev_upload(ctx_->stream, ci));
-            D.lc_val = track(dev_upload(ctx_->stream, cv));
-            upload_row_blocks(nC, cp, D.rb_c, D.nrb_c);
+            D.lc_idx = track(dev_upload(ctx_->stream, ci, kStreamPad));
+            D.lc_val = track(dev_upload(ctx_->stream, cv, kStreamPad));
+            D.st_c = upload_stream(nC, cp, ci);
             D.wc = pick_lanes((long)ci.size(), nC);
             D.wf = D.wb = pick_lanes((long)bi.size(), nB);
             transpose(nC, nB, cp, ci, cv, tp, ti, tv);
             D.sct = upload_sell(build_sell(nB, tp, ti, tv, sigma_, true));
             D.lct_ptr = track(dev_upload(ctx_->stream, tp));
-            D.lct_idx = track(dev_upload(ctx_->stream, ti));
-            D.lct_val = track(dev_upload(ctx_->stream, tv));
-            upload_row_blocks(nB, tp, D.rb_ct, D.nrb_ct);
+            D.lct_idx = track(dev_upload(ctx_->stream, ti, kStreamPad));
+            D.lct_val = track(dev_upload(ctx_->stream, tv, kStreamPad));
+            D.st_ct = upload_stream(nB, tp, ti);
             D.wct = pick_lanes((long)ti.size(), nB);
             D.buf = track(dev_alloc<W>(n));
             D.out = track(dev_alloc<W>(n));
@@ -468,9 +469,8 @@ class IldlImpl : public IldlImplBase {
                       W *xout) {
         hipStream_t s = ctx_->stream;
         if (form == 1) {
-            ildl_jacobi_stream<T, W>(s, fwd ? D.nrb_b : D.nrb_t, fwd ? D.rb_b : D.rb_t,
-                                     fwd ? D.lb_ptr : D.lt_ptr, fwd ? D.lb_idx : D.lt_idx,
-                                     fwd ? D.lb_val : D.lt_val, b, xin, xout, xcd_ & 1);
+            ildl_stream<T, W>(s, fwd ? D.st_b : D.st_t, fwd ? D.lb_idx : D.lt_idx,
+                              fwd ? D.lb_val : D.lt_val, xin, b, xout, xcd_ & 1);
         } else if (form > 0) {
             ildl_jacobi_csr<T, W>(s, form, D.nB, fwd ? D.lb_ptr : D.lt_ptr,
                                   fwd ? D.lb_idx : D.lt_idx, fwd ? D.lb_val : D.lt_val, b, xin,
@@ -484,12 +484,8 @@ class IldlImpl : public IldlImplBase {
     void sub_launch(const DevLevel<T, W> &D, bool trans, int form, const W *x, W *y) {
         hipStream_t s = ctx_->stream;
         if (form == 1) {
-            if (trans)
-                ildl_sub_stream<T, W>(s, D.nrb_ct, D.rb_ct, D.lct_ptr, D.lct_idx, D.lct_val, x,
-                                      y, xcd_ & 1);
-            else
-                ildl_sub_stream<T, W>(s, D.nrb_c, D.rb_c, D.lc_ptr, D.lc_idx, D.lc_val, x, y,
-                                      xcd_ & 1);
+            ildl_stream<T, W>(s, trans ? D.st_ct : D.st_c, trans ? D.lct_idx : D.lc_idx,
+                              trans ? D.lct_val : D.lc_val, x, y, y, xcd_ & 1);
         } else if (form > 0) {
             if (trans)
                 ildl_sub_csr<T, W>(s, form, D.nB, D.lct_ptr, D.lct_idx, D.lct_val, x, y,
@@ -571,10 +567,17 @@ class IldlImpl : public IldlImplBase {
         return v;
     }
 
-    void upload_row_blocks(int nrows, const std::vector<int> &ptr, int *&dev, int &nblk) {
-        const std::vector<int> rb = stream_row_blocks(nrows, ptr.data());
-        nblk = (int)rb.size() - 1;
-        dev = track(dev_upload(ctx_->stream, rb));
+    StreamView upload_stream(int nrows, const std::vector<int> &ptr,
+                             const std::vector<int> &idx) {
+        const StreamHost h = build_stream(nrows, ptr, idx);
+        StreamView v;
+        v.nblk = (int)h.desc.size();
+        v.cap = h.cap;
+        v.desc = track(dev_upload(ctx_->stream, h.desc));
+        v.cbase = track(dev_upload(ctx_->stream, h.cbase));
+        v.off = track(dev_upload(ctx_->stream, h.off));
+        v.c16 = track(dev_upload(ctx_->stream, h.c16));
+        return v;
     }
 
     SellDev<T> upload_sell(const SellHost<T> &h) {

@@ -15,6 +15,7 @@
 #include "xcd.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <vector>
 
 namespace jdhip {
@@ -171,38 +172,48 @@ __global__ __launch_bounds__(kB) void k_sub_csr(int nrows, const int *__restrict
     }
 }
 
-// CSR-stream form: block b owns the rows rblk[b] .. rblk[b+1]-1, chosen on
-// the host so that their entries number at most kStreamCap (and rows at most
-// kB), or a single longer row.  The block streams the entries of its rows
-// (consecutive in CSR) with fully coalesced, independent loads, parks the
-// products in LDS, then sums each row with a group of t lanes (t = the power
-// of two that spreads the block's rows over its 256 threads, at most 64) and
-// a butterfly.  A single row longer than kStreamCap is summed by the whole
-// block with strided loads.  Every row of the range is written.
-static constexpr int kStreamCap = 2048;
-
-template <typename T, typename W>
-__device__ __forceinline__ void stream_rows(long blk, const int *__restrict__ rblk,
-                                            const int *__restrict__ ptr,
-                                            const int *__restrict__ idx,
-                                            const T *__restrict__ val,
-                                            const W *__restrict__ x, int &row, double &sum,
-                                            bool &owner) {
-    __shared__ double prod[kStreamCap];
+// CSR-stream form, out = src - M x: a block owns a run of consecutive rows
+// with at most CAP - 2 entries (and at most kB rows), or a single longer row.
+// It streams the entries of its rows (consecutive in CSR) with coalesced,
+// independent loads, parks the products in LDS, then sums each row with a
+// group of t lanes (t = the power of two that spreads the block's rows over
+// its 256 threads, at most 64) and a butterfly.  Every row is written.
+//
+// Bound by memory on large levels and by the chain of dependent loads on
+// small ones, so the chain is kept to three: the block's descriptor; then
+// columns, values, the row's entry range and src together; then the gathers
+// of x.  A thread takes entries in pairs (16 bytes of values, 4 or 8 of
+// columns a load); pairs start at an even entry, so the first may hold an
+// entry of the block before and the last one of the block behind, which are
+// loaded (the arrays end in two spare entries) and not summed.  Columns are
+// 16-bit offsets from the block's smallest column where they span less than
+// 2^16.  Level-1 and level-2 sweeps, before (2048 entries a block, one entry a
+// load, row pointers read in two dependent steps) -> now: 128^3 Laplacian
+// (7.5M and 10.0M entries) 26.4 -> 24.7 and 27.4 -> 27.0 us, 64^3 (1.0M and
+// 1.2M) 7.2 -> 6.0 and 6.9 -> 5.4 us, Anderson L = 32 (609k) 8.1 -> 5.4 us.
+template <int CAP, typename T, typename W>
+__global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restrict__ idx,
+                                               const T *__restrict__ val, const W *x,
+                                               const W *src, W *out, int xcd) {
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double prod[CAP];
     __shared__ double red[kB / 64];
+    constexpr int kPairs = CAP / kB / 2;  // pairs per thread
+    static_assert(kPairs * kB * 2 == CAP, "a block holds kPairs pairs per thread");
+    const long blk = logical_block(xcd);
     const int tid = threadIdx.x;
-    const int r0 = rblk[blk], r1 = rblk[blk + 1];
-    const int e0 = ptr[r0], e1 = ptr[r1];
-    const int ne = e1 - e0;
-    owner = false;
-    if (r1 - r0 == 1 && ne > kStreamCap) {  // one long row
+    const int4 d = M.desc[blk];
+    const int cb = M.cbase[blk];
+    const int r0 = d.x, nr = d.y & 0xffff, e0 = d.z, ne = d.w;
+    const bool narrow = d.y >> 16;
+    if (ne > CAP - 2) {  // one long row
         double s0 = 0.0, s1 = 0.0;
         int k = e0 + tid;
-        for (; k + kB < e1; k += 2 * kB) {
+        for (; k + kB < e0 + ne; k += 2 * kB) {
             s0 += (double)val[k] * (double)x[idx[k]];
             s1 += (double)val[k + kB] * (double)x[idx[k + kB]];
         }
-        if (k < e1) s0 += (double)val[k] * (double)x[idx[k]];
+        if (k < e0 + ne) s0 += (double)val[k] * (double)x[idx[k]];
         double s = s0 + s1;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -212,76 +223,71 @@ __device__ __forceinline__ void stream_rows(long blk, const int *__restrict__ rb
             double t = 0.0;
 #pragma unroll
             for (int w = 0; w < kB / 64; ++w) t += red[w];
-            row = r0;
-            sum = t;
-            owner = true;
+            out[r0] = (W)((double)src[r0] - t);
         }
         return;
     }
-    // ne <= kStreamCap and r1 - r0 <= kB by construction of rblk.  A thread
-    // takes the entries tid, tid + kB, ...: all their column indices are
-    // loaded first, then the values and the gathers of x, so that each wave
-    // has up to 3 x kPer loads in flight rather than one index and one
-    // gather at a time.  Positions past the block's entries load its last
-    // entry again (in bounds, branch-free) and are not stored.
-    constexpr int kPer = kStreamCap / kB;
-    static_assert(kPer * kB == kStreamCap, "stream blocks hold kPer entries per thread");
-    if (ne > 0) {
-        const int last = ne - 1;
-        int ci[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) ci[u] = idx[e0 + min(tid + u * kB, last)];
-        double pv[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u)
-            pv[u] = (double)val[e0 + min(tid + u * kB, last)] * (double)x[ci[u]];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u)
-            if (tid + u * kB < ne) prod[tid + u * kB] = pv[u];
-    }
-    __syncthreads();
-    const int nr = r1 - r0;
     int t = 64;
     while (t > 1 && t * nr > kB) t >>= 1;
     const int g = tid / t, l = tid % t;
-    double s = 0.0;
-    if (g < nr) {
-        const int a = ptr[r0 + g] - e0, b = ptr[r0 + g + 1] - e0;
-        for (int k = a + l; k < b; k += t) s += prod[k];
+    const bool mine = g < nr;
+    int a = 0, b = 0;
+    double sv = 0.0;
+    if (mine) {
+        const unsigned short *o = M.off + (r0 + blk + g);
+        a = o[0];
+        b = o[1];
+        if (l == 0) sv = (double)src[r0 + g];
     }
+    const int ea = e0 & ~1, sh = e0 & 1, tot = ne + sh;  // entries from the even start on
+    if (ne > 0) {
+        const int last = (tot + 1) / 2 - 1;
+        int c0[kPairs], c1[kPairs];
+        T v0[kPairs], v1[kPairs];
+        if (narrow) {
+            const ushort2 *c = (const ushort2 *)(M.c16 + ea);
+#pragma unroll
+            for (int u = 0; u < kPairs; ++u) {
+                const ushort2 q = c[min(tid + u * kB, last)];
+                c0[u] = cb + q.x;
+                c1[u] = cb + q.y;
+            }
+        } else {
+            const int2 *c = (const int2 *)(idx + ea);
+#pragma unroll
+            for (int u = 0; u < kPairs; ++u) {
+                const int2 q = c[min(tid + u * kB, last)];
+                c0[u] = q.x;
+                c1[u] = q.y;
+            }
+        }
+        const T2 *v = (const T2 *)(val + ea);
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            const T2 q = v[min(tid + u * kB, last)];
+            v0[u] = q.x;
+            v1[u] = q.y;
+        }
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            // threads past the end repeat the last pair; an entry that is not
+            // the block's own takes its partner's column (a narrow offset
+            // holds from its own block's base only)
+            const int k = 2 * min(tid + u * kB, last);
+            if (k < sh) c0[u] = c1[u];
+            if (k + 1 >= tot) c1[u] = c0[u];
+            double2 p;
+            p.x = (double)v0[u] * (double)x[c0[u]];
+            p.y = (double)v1[u] * (double)x[c1[u]];
+            if (tid + u * kB <= last) *(double2 *)(prod + k) = p;
+        }
+    }
+    __syncthreads();
+    double s = 0.0;
+    if (mine)
+        for (int k = sh + a + l; k < sh + b; k += t) s += prod[k];
     for (int o = t / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, t);
-    if (g < nr && l == 0) {
-        row = r0 + g;
-        sum = s;
-        owner = true;
-    }
-}
-
-template <typename T, typename W>
-__global__ __launch_bounds__(kB) void k_jacobi_stream(const int *__restrict__ rblk,
-                                                      const int *__restrict__ ptr,
-                                                      const int *__restrict__ idx,
-                                                      const T *__restrict__ val, const W *b,
-                                                      const W *xin, W *xout, int xcd) {
-    int row = 0;
-    double s = 0.0;
-    bool owner = false;
-    stream_rows(logical_block(xcd), rblk, ptr, idx, val, xin, row, s, owner);
-    if (owner) xout[row] = (W)((double)b[row] - s);
-}
-
-template <typename T, typename W>
-__global__ __launch_bounds__(kB) void k_sub_stream(const int *__restrict__ rblk,
-                                                   const int *__restrict__ ptr,
-                                                   const int *__restrict__ idx,
-                                                   const T *__restrict__ val,
-                                                   const W *__restrict__ x, W *__restrict__ y,
-                                                   int xcd) {
-    int row = 0;
-    double s = 0.0;
-    bool owner = false;
-    stream_rows(logical_block(xcd), rblk, ptr, idx, val, x, row, s, owner);
-    if (owner) y[row] = (W)((double)y[row] - s);
+    if (mine && l == 0) out[r0 + g] = (W)(sv - s);
 }
 
 template <typename W>
@@ -395,40 +401,48 @@ void ildl_sub_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *
 #undef JDHIP_SC
 }
 template <typename T, typename W>
-void ildl_jacobi_stream(hipStream_t s, int nblk, const int *rblk, const int *ptr,
-                        const int *idx, const T *val, const W *b, const W *xin, W *xout,
-                        int xcd) {
-    if (nblk <= 0) return;
-    k_jacobi_stream<T, W><<<nblk, kB, 0, s>>>(rblk, ptr, idx, val, b, xin, xout, xcd);
+void ildl_stream(hipStream_t s, const StreamView &M, const int *idx, const T *val, const W *x,
+                 const W *src, W *out, int xcd) {
+    if (M.nblk <= 0) return;
+    if (M.cap == 512)
+        k_stream<512, T, W><<<M.nblk, kB, 0, s>>>(M, idx, val, x, src, out, xcd);
+    else
+        k_stream<1024, T, W><<<M.nblk, kB, 0, s>>>(M, idx, val, x, src, out, xcd);
 }
-template <typename T, typename W>
-void ildl_sub_stream(hipStream_t s, int nblk, const int *rblk, const int *ptr, const int *idx,
-                     const T *val, const W *x, W *y, int xcd) {
-    if (nblk <= 0) return;
-    k_sub_stream<T, W><<<nblk, kB, 0, s>>>(rblk, ptr, idx, val, x, y, xcd);
-}
-std::vector<int> stream_row_blocks(int nrows, const int *ptr) {
-    std::vector<int> rb;
-    rb.push_back(0);
+
+// Entries a block holds: 1024 where that leaves enough blocks for the 256 CUs,
+// else 512.  Measured (us a sweep, 512 against 1024): 354k entries 3.8 / 4.1,
+// 609k 5.4 / 5.8, 988k 6.3 / 6.0, 1.2M 5.8 / 5.4, 7.5M 28.7 / 24.7.
+static constexpr long kStreamWide = 800000;
+
+StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx) {
+    StreamHost h;
+    const int nnz = ptr[nrows];
+    h.cap = nnz >= kStreamWide ? 1024 : 512;
+    const int most = h.cap - 2;  // a block may start one entry before its own
+    h.c16.assign((size_t)nnz + kStreamPad, 0);
     int r = 0;
     while (r < nrows) {
-        const int len = ptr[r + 1] - ptr[r];
-        if (len > kStreamCap) {  // a long row alone
-            ++r;
-            rb.push_back(r);
-            continue;
+        const int r0 = r, e0 = ptr[r];
+        while (r < nrows && r - r0 < kB && ptr[r + 1] - e0 <= most) ++r;
+        if (r == r0) ++r;  // a long row alone
+        const int ne = ptr[r] - e0;
+        int cmin = INT_MAX, cmax = INT_MIN;
+        for (int k = e0; k < e0 + ne; ++k) {
+            cmin = std::min(cmin, idx[k]);
+            cmax = std::max(cmax, idx[k]);
         }
-        int e = 0, cnt = 0;
-        while (r < nrows && cnt < kB) {
-            const int l = ptr[r + 1] - ptr[r];
-            if (l > kStreamCap || e + l > kStreamCap) break;
-            e += l;
-            ++cnt;
-            ++r;
-        }
-        rb.push_back(r);
+        if (cmin > cmax) cmin = cmax = 0;
+        const bool narrow = (long)cmax - cmin < 65536;
+        if (narrow)
+            for (int k = e0; k < e0 + ne; ++k) h.c16[k] = (unsigned short)(idx[k] - cmin);
+        h.desc.push_back(make_int4(r0, (r - r0) | (narrow ? 1 << 16 : 0), e0, ne));
+        h.cbase.push_back(narrow ? cmin : 0);
+        // entry range of each row, from the block's first entry (a long row's
+        // range is not read)
+        for (int i = r0; i <= r; ++i) h.off.push_back((unsigned short)(ptr[i] - e0));
     }
-    return rb;
+    return h;
 }
 
 template <typename W>
@@ -478,11 +492,8 @@ void ildl_dense_gemv(hipStream_t s, int m, const T *Minv, const W *x, W *y) {
     template void ildl_sub_csr<T, W>(hipStream_t, int, int, const int *, const int *,         \
                                      const T *, const W *, W *, int);                        \
     template void ildl_dense_gemv<T, W>(hipStream_t, int, const T *, const W *, W *);         \
-    template void ildl_jacobi_stream<T, W>(hipStream_t, int, const int *, const int *,        \
-                                           const int *, const T *, const W *, const W *,      \
-                                           W *, int);                                         \
-    template void ildl_sub_stream<T, W>(hipStream_t, int, const int *, const int *,           \
-                                        const int *, const T *, const W *, W *, int);
+    template void ildl_stream<T, W>(hipStream_t, const StreamView &, const int *, const T *,   \
+                                    const W *, const W *, W *, int);
 INST(double, double)
 INST(float, double)
 INST(float, float)

@@ -63,18 +63,34 @@ void ildl_sub_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *
 // y[r] -= sum_j M(r, j) x[j] over the rows of a SELL-C-sigma matrix
 template <typename T, typename W>
 void ildl_sub_sell(hipStream_t s, const SellView &M, const T *val, const W *x, W *y, int xcd);
-// CSR-stream form: blocks of consecutive rows with at most 2048 entries
-// (and 256 rows) each, or one longer row; rblk[b] = first row of block b,
-// rblk[nblk] = nrows.  Entries are streamed through LDS with coalesced loads.
+// CSR-stream form: blocks of consecutive rows with at most cap - 2 entries
+// (and 256 rows) each, or one longer row, streamed through LDS with coalesced
+// loads.  The product reads the CSR's own values and columns (which end in
+// kStreamPad spare entries, allocated and zero) beside this view:
+// desc[b] = {first row, rows + 2^16 when narrow, first entry, entries};
+// cbase[b] + c16[entry] is a narrow block's column; off[row + b] and the next
+// are a row's entry range from the block's first entry.
+constexpr int kStreamPad = 2;
+struct StreamView {
+    int nblk = 0;
+    int cap = 1024;
+    const int4 *desc = nullptr;
+    const int *cbase = nullptr;
+    const unsigned short *off = nullptr;
+    const unsigned short *c16 = nullptr;
+};
+struct StreamHost {
+    int cap = 1024;
+    std::vector<int4> desc;
+    std::vector<int> cbase;
+    std::vector<unsigned short> off, c16;
+};
+StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx);
+// out = src - M x over every row (a sweep: src = b; a product: src = out = y).
 // xcd != 0: every XCD takes one contiguous range of row blocks.
-std::vector<int> stream_row_blocks(int nrows, const int *ptr);
 template <typename T, typename W>
-void ildl_jacobi_stream(hipStream_t s, int nblk, const int *rblk, const int *ptr,
-                        const int *idx, const T *val, const W *b, const W *xin, W *xout,
-                        int xcd);
-template <typename T, typename W>
-void ildl_sub_stream(hipStream_t s, int nblk, const int *rblk, const int *ptr, const int *idx,
-                     const T *val, const W *x, W *y, int xcd);
+void ildl_stream(hipStream_t s, const StreamView &M, const int *idx, const T *val, const W *x,
+                 const W *src, W *out, int xcd);
 template <typename W>
 void ildl_dscale(hipStream_t s, int n, const double *dinv, W *x);
 // x = D^-1 x with 2x2 blocks: row i pairs with pair[i] (-1: 1x1 pivot,

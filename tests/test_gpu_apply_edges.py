@@ -1,0 +1,66 @@
+"""The preconditioner apply's kernels at the sizes where they can go wrong,
+against the oracle's apply on the same factor.
+
+Tolerance: both sides sum the same products in double in another order; the
+existing parity bar of the FP64 apply (1e-12 relative) holds throughout.
+"""
+import numpy as np
+import pytest
+
+from jadamilu_amd import matrices as M
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _hub(n, k):
+    """A path of n nodes and a hub coupled to the last k of them (SPD): the
+    coupling block holds a row of about k entries."""
+    r = np.arange(n - 1)
+    c = np.arange(n - k, n)
+    diag = np.full(n + 1, 4.0)
+    diag[-1] = 2.0 * n
+    rows, cols = np.concatenate([r, c]), np.concatenate([r + 1, np.full(k, n)])
+    return M.from_pairs(n + 1, rows, cols, -np.ones(rows.size), diag)
+
+
+def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=300):
+    from jadamilu_amd.ildl import IldlFactor
+    from jadamilu_amd.jd import Context
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    ia, ja, a = gen()
+    n = ia.size - 1
+    f = IldlFactor(n, ia, ja, a, droptol=1e-3, spd=spd, single=single, dense_max=dense_max,
+                   coupling=coupling)
+    assert f.ierr == 0
+    ctx = Context(0)
+    for name, value in options.items():
+        ctx.set_option(name, value)
+    ctx.attach_ildl(f, sweeps=sweeps)
+    ex = f.export()
+    rng = np.random.default_rng(3)
+    for _ in range(2):
+        r = rng.standard_normal(n)
+        rd = torch.tensor(r, device="cuda:0")
+        zd = torch.full_like(rd, float("nan"))
+        torch.cuda.synchronize()
+        ctx.precond_apply(zd.data_ptr(), rd.data_ptr())
+        torch.cuda.synchronize()
+        zo = O.ildl_apply(ex, r, sweeps=sweeps)
+        tol = 2e-5 if single else 1e-12
+        assert np.linalg.norm(zd.cpu().numpy() - zo) <= tol * np.linalg.norm(zo)
+    ctx.close()
+
+
+# rows around the 510 entries that a block of the small CSR-stream form holds
+@pytest.mark.parametrize("k", [508, 509, 510, 511, 512, 513])
+@pytest.mark.parametrize("single", [False, True])
+def test_stream_rows_at_the_block_size(k, single):
+    _check(lambda: _hub(700, k), {"ildl_form": 1}, 3, single=single)
+
+
+# a level large enough for the blocks of 1022 entries
+def test_stream_wide_blocks():
+    _check(lambda: M.laplace((64, 63, 61)), {"ildl_form": 1}, 2)
