@@ -205,7 +205,7 @@ def bench_batch(args, params, neig, madspace, isearch, sigma, mem):
                           madspace=madspace, maxiter=args.maxiter, tol=args.tol,
                           droptol=args.droptol, mem=mem, icntl=(0, 0, 0, 0, 1)))
     print(f"# batch of {count} problems, total n {ntot}", file=sys.stderr, flush=True)
-    bopts = {}  # (graph replay is not offered by the batch driver)
+    bopts = {}  # (the batch driver's workers choose graph replay by themselves)
     for kv in args.set:
         name, value = kv.split("=", 1)
         bopts[name] = float(value)
@@ -496,7 +496,8 @@ def main():
     ap.add_argument("--inner32", action="store_true",
                     help="with --single: run the inner solver in FP32 as well")
     ap.add_argument("--graph", action="store_true",
-                    help="replay the preconditioner apply from captured HIP graphs")
+                    help="replay the preconditioner apply from a HIP graph (the default where it "
+                         "holds few enough launches)")
     ap.add_argument("--set", action="append", default=[], metavar="NAME=VALUE",
                     help="extra jdhip_set_option(NAME, VALUE), repeatable")
     ap.add_argument("--batch-count", type=int, default=0,
@@ -579,7 +580,8 @@ def main():
     icntl = (0, -1, 0, 0, single)  # timed solves: keep the resident factor
     ctx.set_option("ildl_sweeps", args.sweeps)
     ctx.set_option("inner_fp32", 1 if args.inner32 else 0)
-    ctx.set_option("ildl_graph", 1 if args.graph else 0)
+    if args.graph:
+        ctx.set_option("ildl_graph", 1)
     for kv in args.set:  # again: they override the flags above
         name, value = kv.split("=", 1)
         ctx.set_option(name, float(value))

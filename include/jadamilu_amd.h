@@ -287,9 +287,8 @@ typedef struct {
 int jdhip_pjd_batch(int device, int nitems, jdhip_batch_item *items, int nworkers);
 /* jdhip_pjd_batch with options (jdhip_set_option names and values) applied
  * to every worker context after the batch's own settings, e.g.
- * "ildl_sweeps" or "ildl_tune_tol".  "ildl_graph" 1 is refused (-1): while
- * one worker captures a graph, another worker's allocations may
- * synchronise the device and invalidate the capture.  An option that
+ * "ildl_sweeps" or "ildl_tune_tol".  "ildl_graph" 1 is refused (-1): the
+ * workers choose by themselves.  An option that
  * jdhip_set_option rejects leaves every item with INFO = -54330. */
 int jdhip_pjd_batch_opts(int device, int nitems, jdhip_batch_item *items, int nworkers,
                          int nopts, const char *const *names, const double *values);
@@ -349,7 +348,8 @@ int jdhip_tall_gemm(jdhip_ctx *ctx, long n, int k, int j, const double *v_dev, l
  * two solves with B per level, as the reference, the default; 1 = L_CB blocks,
  * see jdhip_ildl_coupling), "ildl_dense_max" (largest final
  * level factored densely), "spmv_lanes", "ildl_graph" (1: replay the
- * preconditioner apply from captured HIP graphs; default 0), "ildl_storage",
+ * preconditioner apply from a HIP graph where it holds at most 1024 launches;
+ * 0: launch it kernel by kernel; default -1, as 1), "ildl_storage",
  * "ildl_xcd", "ildl_sigma" (device layout of the factor), "ildl_threads"
  * (host threads of the factorization), "sync_blocking" (1: the iteration's
  * waits for the device sleep on a blocking-sync event instead of spinning;

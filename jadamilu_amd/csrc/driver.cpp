@@ -71,12 +71,9 @@ struct Solver {
     // 128^3 Laplacian: 1.47 ms against 1.84 ms for factor order / window 1024)
     int ildl_storage = 1, ildl_xcd = 1;
     int ildl_sigma = 256;
-    // replay the preconditioner apply from captured HIP graphs: off by default
-    // (no gain measured on the 128^3 Laplacian, whose apply is bandwidth- and
-    // not launch-bound; and a capture on one worker's stream is invalidated by
-    // synchronous HIP calls of other threads in the batched driver, whose
-    // blocking streams synchronise with the null stream)
-    bool ildl_graph = false;
+    // replay the preconditioner apply from a HIP graph: 0 never, 1 and -1 where
+    // the apply holds few enough launches (ildl.cpp)
+    int ildl_graph = -1;
     int ildl_threads = 0;  // host threads of the factorisation (0: all cores, <= 16)
     int ildl_vec32 = -1;   // FP32 factor: work vectors FP32 (1), FP64 (0), by definiteness (-1)
     bool ildl_autotune = true;  // kernel form of each product by timing at set-up
@@ -1272,7 +1269,7 @@ int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value) {
         S.ildl_form = f;
     }
     else if (k == "ildl_graph") {
-        S.ildl_graph = value != 0.0;
+        S.ildl_graph = (int)value;
         if (S.ildl && S.ildl->ready()) S.ildl->impl()->set_graphs(S.ildl_graph);
     }
     else return -2;

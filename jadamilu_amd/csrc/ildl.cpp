@@ -258,7 +258,7 @@ class IldlImpl : public IldlImplBase {
           sigma_(sigma) {}
     ~IldlImpl() override {
         hipStreamSynchronize(ctx_->stream);
-        clear_graphs();
+        clear_graph();
         for (void *p : allocs_) hipFree(p);
     }
 
@@ -431,9 +431,7 @@ class IldlImpl : public IldlImplBase {
     }
 
     // Triangular solve with L_B (fwd) or L_B^T in place on x (nB entries).
-    void tri_solve(const DevLevel<T, W> &D, bool fwd) { tri_solve(D, fwd, D.buf); }
-    void tri_solve(const DevLevel<T, W> &D, bool fwd, W *x) {
-        hipStream_t s = ctx_->stream;
+    void tri_solve(const Put &s, const DevLevel<T, W> &D, bool fwd, W *x) {
         const int *ptr = fwd ? D.lb_ptr : D.lt_ptr;
         const int *idx = fwd ? D.lb_idx : D.lt_idx;
         const T *val = fwd ? D.lb_val : D.lt_val;
@@ -455,19 +453,17 @@ class IldlImpl : public IldlImplBase {
         for (int k = 0; k < nsw; ++k) {
             const bool last = (k == nsw - 1) && nsw >= 2;
             W *xout = last ? x : bufs[k & 1];
-            sweep_launch(D, fwd, lanes, x, xin, xout);
+            sweep_launch(s, D, fwd, lanes, x, xin, xout);
             xin = xout;
         }
-        if (nsw == 1)
-            JDHIP_CHECK(hipMemcpyAsync(x, D.t1, sizeof(W) * D.nB, hipMemcpyDeviceToDevice, s));
+        if (nsw == 1) ildl_copy<W>(s, D.nB, D.t1, x);
     }
 
     // One Jacobi sweep xout = b - N xin of the level's L_B (fwd) or L_B^T,
     // in the given kernel form: 0 one lane per row on the SELL-C-sigma copy,
     // else CSR with that many lanes per row.
-    void sweep_launch(const DevLevel<T, W> &D, bool fwd, int form, const W *b, const W *xin,
-                      W *xout) {
-        hipStream_t s = ctx_->stream;
+    void sweep_launch(const Put &s, const DevLevel<T, W> &D, bool fwd, int form, const W *b,
+                      const W *xin, W *xout) {
         if (form == 1) {
             ildl_stream<T, W>(s, fwd ? D.st_b : D.st_t, fwd ? D.lb_idx : D.lt_idx,
                               fwd ? D.lb_val : D.lt_val, xin, b, xout, xcd_ & 1);
@@ -481,8 +477,8 @@ class IldlImpl : public IldlImplBase {
         }
     }
     // y -= L_CB x (C rows; trans = false) or y -= L_CB^T x (B rows)
-    void sub_launch(const DevLevel<T, W> &D, bool trans, int form, const W *x, W *y) {
-        hipStream_t s = ctx_->stream;
+    void sub_launch(const Put &s, const DevLevel<T, W> &D, bool trans, int form, const W *x,
+                    W *y) {
         if (form == 1) {
             ildl_stream<T, W>(s, trans ? D.st_ct : D.st_c, trans ? D.lct_idx : D.lc_idx,
                               trans ? D.lct_val : D.lc_val, x, y, y, xcd_ & 1);
@@ -539,22 +535,22 @@ class IldlImpl : public IldlImplBase {
             JDHIP_CHECK(hipMemsetAsync(D.t1, 0, sizeof(W) * std::max(D.nB, 1), s));
             JDHIP_CHECK(hipMemsetAsync(D.t2, 0, sizeof(W) * std::max(D.nB, 1), s));
             if (D.nB > 0) {
-                D.wf = best([&](int f) { sweep_launch(D, true, f, D.buf, D.t1, D.t2); });
-                D.wb = best([&](int f) { sweep_launch(D, false, f, D.buf, D.t1, D.t2); });
+                D.wf = best([&](int f) { sweep_launch(s, D, true, f, D.buf, D.t1, D.t2); });
+                D.wb = best([&](int f) { sweep_launch(s, D, false, f, D.buf, D.t1, D.t2); });
             }
             if (D.nC > 0) {
-                D.wc = best([&](int f) { sub_launch(D, false, f, D.buf, D.buf + D.nB); });
-                D.wct = best([&](int f) { sub_launch(D, true, f, D.out, D.buf); });
+                D.wc = best([&](int f) { sub_launch(s, D, false, f, D.buf, D.buf + D.nB); });
+                D.wct = best([&](int f) { sub_launch(s, D, true, f, D.out, D.buf); });
             }
         }
         JDHIP_CHECK(hipStreamSynchronize(s));
         hipEventDestroy(e0);
         hipEventDestroy(e1);
-        clear_graphs();
+        clear_graph();
     }
     void set_forms(int form) override {
         for (auto &D : lv_) D.wf = D.wb = D.wc = D.wct = form;
-        clear_graphs();
+        clear_graph();
     }
     std::vector<int> level_forms() const override {
         std::vector<int> v;
@@ -601,7 +597,7 @@ class IldlImpl : public IldlImplBase {
     void set_all(int k) {
         sweeps_ = k;
         for (auto &D : lv_) D.k = k;
-        clear_graphs();
+        clear_graph();
     }
 
     int tune_sweeps(double tol, bool by_time) override {
@@ -695,7 +691,7 @@ class IldlImpl : public IldlImplBase {
             set_all(0);
         }
         tuning_ = false;
-        clear_graphs();
+        clear_graph();
         hipEventDestroy(e0);
         hipEventDestroy(e1);
         hipFree(r);
@@ -709,112 +705,134 @@ class IldlImpl : public IldlImplBase {
         return v;
     }
 
-    void apply(double *z, const double *r) override { apply_cached<double>(z, r); }
-    void apply_f(float *z, const float *r) override { apply_cached<float>(z, r); }
+    void apply(double *z, const double *r) override { apply_any<double>(z, r); }
+    void apply_f(float *z, const float *r) override { apply_any<float>(z, r); }
 
-    // The apply is a fixed sequence of 30-100 launches (more in the exact
-    // mode); it is captured once per (output, input) pair into a HIP graph
-    // and replayed with a single launch.  The sequence records kernels and
-    // device-to-device copies only.  Any change of the sweep setting drops
-    // the cached graphs; tuning runs uncached.
+    // The apply is a fixed sequence of some tens to hundreds of launches, most
+    // of them shorter than the 2.5-4.5 us that the host takes to enqueue one
+    // (a graph's node takes 1.6-1.9 us).  Everything between the first gather
+    // and the last scatter works on the factor's own vectors, so it is built
+    // once per factor into a HIP graph and replayed for any input and output.
+    // Exact solves (a launch per dependency level) can have 10^5 launches and
+    // keep to the stream, as does everything on a stream under capture, which
+    // cannot take a graph launch.
     template <typename TV>
-    void apply_cached(TV *z, const TV *r) {
-        if (!graphs_on_ || tuning_) {
-            apply_io<TV>(z, r);
-            return;
-        }
-        const int type = sizeof(TV) == 8 ? 0 : 1;
-        for (auto &g : graphs_)
-            if (g.z == (const void *)z && g.r == (const void *)r && g.type == type) {
-                JDHIP_CHECK(hipGraphLaunch(g.exec, ctx_->stream));
-                return;
-            }
-        if (graphs_.size() >= 16) {  // unexpected variety of buffers: no caching
-            apply_io<TV>(z, r);
-            return;
-        }
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t exec = nullptr;
-        JDHIP_CHECK(hipStreamBeginCapture(ctx_->stream, hipStreamCaptureModeThreadLocal));
-        apply_io<TV>(z, r);
-        JDHIP_CHECK(hipStreamEndCapture(ctx_->stream, &graph));
-        JDHIP_CHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-        JDHIP_CHECK(hipGraphDestroy(graph));
-        graphs_.push_back({(const void *)z, (const void *)r, type, exec});
-        JDHIP_CHECK(hipGraphLaunch(exec, ctx_->stream));
+    void apply_any(TV *z, const TV *r) {
+        const Put q(ctx_->stream);
+        const bool replay = graph_ && !tuning_ && !capturing();
+        head<TV>(q, r);
+        if (replay) JDHIP_CHECK(hipGraphLaunch(graph_, ctx_->stream));
+        else body(q);
+        tail<TV>(q, z);
     }
-    void clear_graphs() {
-        for (auto &g : graphs_) hipGraphExecDestroy(g.exec);
-        graphs_.clear();
+    bool capturing() const {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        JDHIP_CHECK(hipStreamIsCapturing(ctx_->stream, &st));
+        return st != hipStreamCaptureStatusNone;
     }
-    void set_graphs(bool on) override {
-        graphs_on_ = on;
-        clear_graphs();
+    // launches of body() with sweeps (exact solves: one per dependency level)
+    long body_launches() const {
+        long c = 0;
+        for (const auto &D : lv_) {
+            const long half = D.k > 0 ? 2 * (D.k + 1)
+                                      : (long)D.fwd_ptr.size() + (long)D.bwd_ptr.size();
+            c += 8 + half * ((fform() && D.nC > 0) ? 2 : 1);
+        }
+        return c;
+    }
+    void clear_graph() {
+        if (!graph_) return;
+        hipStreamSynchronize(ctx_->stream);
+        hipGraphExecDestroy(graph_);
+        graph_ = nullptr;
+    }
+    void set_graphs(int mode) override {
+        clear_graph();
+        if (mode == 0 || lv_.empty() || body_launches() > kGraphMax) return;
+        hipGraph_t g = nullptr;
+        JDHIP_CHECK(hipGraphCreate(&g, 0));
+        try {
+            body(Put(g));
+            JDHIP_CHECK(hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0));
+        } catch (...) {
+            hipGraphDestroy(g);
+            throw;
+        }
+        JDHIP_CHECK(hipGraphDestroy(g));
     }
 
     template <typename TV>
-    void apply_io(TV *z, const TV *r) {
-        hipStream_t s = ctx_->stream;
-        const int L = (int)lv_.size();
-        if (L == 0) {
-            // only a dense level: z = Minv r
-            ildl_gather<TV, W>(s, f_.m, ident_(), ones_(), r, dx_);
-            ildl_dense_gemv<T, W>(s, f_.m, dmat_, dx_, dy_);
+    void head(const Put &s, const TV *r) {
+        if (lv_.empty()) ildl_gather<TV, W>(s, f_.m, ident_(), ones_(), r, dx_);
+        else ildl_gather<TV, W>(s, lv_[0].n, lv_[0].perm, lv_[0].scal, r, lv_[0].buf);
+    }
+    template <typename TV>
+    void tail(const Put &s, TV *z) {
+        if (lv_.empty()) {
             ildl_scatter<W, TV>(s, f_.m, f_.m, ident_(), ones_(), dy_, dy_, z);
+            return;
+        }
+        const DevLevel<T, W> &D = lv_[0];
+        ildl_scatter<W, TV>(s, D.n, D.nB, D.perm, D.scal, D.buf, coarse_of(0), z);
+    }
+    // x_C of level l: the next level's result, or the dense level's
+    const W *coarse_of(int l) const {
+        return l + 1 < (int)lv_.size() ? lv_[l + 1].out : dy_;
+    }
+    void body(const Put &s) {
+        const int L = (int)lv_.size();
+        if (L == 0) {  // only a dense level: z = Minv r
+            ildl_dense_gemv<T, W>(s, f_.m, dmat_, dx_, dy_);
             return;
         }
         for (int l = 0; l < L; ++l) {
             DevLevel<T, W> &D = lv_[l];
-            if (l == 0) ildl_gather<TV, W>(s, D.n, D.perm, D.scal, r, D.buf);
-            else {
+            if (l > 0) {
                 const DevLevel<T, W> &P = lv_[l - 1];
                 ildl_gather<W, W>(s, D.n, D.perm, D.scal, P.buf + P.nB, D.buf);
             }
-            tri_solve(D, true);
+            tri_solve(s, D, true, D.buf);
             if (fform()) {
                 // y_B = B^-1 b_B, then b_C -= F^T y_B
-                dscale(D, D.buf);
-                tri_solve(D, false);
-                if (D.nC > 0) sub_launch(D, false, D.wc, D.buf, D.buf + D.nB);
+                dscale(s, D, D.buf);
+                tri_solve(s, D, false, D.buf);
+                if (D.nC > 0) sub_launch(s, D, false, D.wc, D.buf, D.buf + D.nB);
             } else {
-                if (D.nC > 0) sub_launch(D, false, D.wc, D.buf, D.buf + D.nB);
-                dscale(D, D.buf);
+                if (D.nC > 0) sub_launch(s, D, false, D.wc, D.buf, D.buf + D.nB);
+                dscale(s, D, D.buf);
             }
         }
-        const W *zc = nullptr;
         if (f_.m > 0) {
             const DevLevel<T, W> &P = lv_[L - 1];
             ildl_dense_gemv<T, W>(s, f_.m, dmat_, P.buf + P.nB, dy_);
-            zc = dy_;
         }
         for (int l = L - 1; l >= 0; --l) {
             DevLevel<T, W> &D = lv_[l];
+            const W *zc = coarse_of(l);
             if (fform()) {
                 if (D.nC > 0) {
                     // x_B = y_B - B^-1 F x_C; D.out is free until the scatter
                     W *t = D.out;
                     ildl_zero<W>(s, D.nB, t);
-                    sub_launch(D, true, D.wct, zc, t);
-                    tri_solve(D, true, t);
-                    dscale(D, t);
-                    tri_solve(D, false, t);
+                    sub_launch(s, D, true, D.wct, zc, t);
+                    tri_solve(s, D, true, t);
+                    dscale(s, D, t);
+                    tri_solve(s, D, false, t);
                     ildl_add<W>(s, D.nB, t, D.buf);
                 }
             } else {
-                if (D.nC > 0) sub_launch(D, true, D.wct, zc, D.buf);
-                tri_solve(D, false);
+                if (D.nC > 0) sub_launch(s, D, true, D.wct, zc, D.buf);
+                tri_solve(s, D, false, D.buf);
             }
-            if (l == 0) ildl_scatter<W, TV>(s, D.n, D.nB, D.perm, D.scal, D.buf, zc, z);
-            else ildl_scatter<W, W>(s, D.n, D.nB, D.perm, D.scal, D.buf, zc, D.out);
-            zc = D.out;
+            if (l > 0) ildl_scatter<W, W>(s, D.n, D.nB, D.perm, D.scal, D.buf, zc, D.out);
         }
     }
 
     bool fform() const { return f_.coupling == 0; }
     // x_B = D^-1 x_B (1x1 and 2x2 pivots)
-    void dscale(const DevLevel<T, W> &D, W *x) {
-        if (D.dpair) ildl_dscale2<W>(ctx_->stream, D.nB, D.dinv, D.doinv, D.dpair, x);
-        else ildl_dscale<W>(ctx_->stream, D.nB, D.dinv, x);
+    void dscale(const Put &s, const DevLevel<T, W> &D, W *x) {
+        if (D.dpair) ildl_dscale2<W>(s, D.nB, D.dinv, D.doinv, D.dpair, x);
+        else ildl_dscale<W>(s, D.nB, D.dinv, x);
     }
     int nlevels() const override { return (int)f_.levels.size(); }
     int dense_m() const override { return f_.m; }
@@ -880,7 +898,7 @@ class IldlImpl : public IldlImplBase {
         hipEvent_t e0, e1;
         JDHIP_CHECK(hipEventCreate(&e0));
         JDHIP_CHECK(hipEventCreate(&e1));
-        auto one = [&]() { sweep_launch(D, true, D.wf, D.buf, D.t1, D.t2); };
+        auto one = [&]() { sweep_launch(s, D, true, D.wf, D.buf, D.t1, D.t2); };
         one();
         JDHIP_CHECK(hipEventRecord(e0, s));
         for (int i = 0; i < reps; ++i) one();
@@ -920,13 +938,11 @@ class IldlImpl : public IldlImplBase {
 
     DevCtx *ctx_;
     IldlMultilevel<T> f_;
-    struct CachedGraph {
-        const void *z, *r;
-        int type;
-        hipGraphExec_t exec;
-    };
-    std::vector<CachedGraph> graphs_;
-    bool graphs_on_ = false, tuning_ = false;
+    // launches that one graph holds at most (exact solves of small factors
+    // included); larger applies are bound by their kernels
+    static constexpr long kGraphMax = 1024;
+    hipGraphExec_t graph_ = nullptr;
+    bool tuning_ = false;
     int sweeps_;
     int storage_;  // 0: factor order, 1: original-index order per level
     int xcd_;      // XCD-contiguous block order in the SELL kernels

@@ -68,8 +68,9 @@ class IldlImplBase {
     // per level: forms of the forward sweep, backward sweep, L_CB, L_CB^T
     // (0 SELL, 1 CSR-stream, k >= 4 lanes per row CSR)
     virtual std::vector<int> level_forms() const = 0;
-    // replay the apply from captured HIP graphs (default on)
-    virtual void set_graphs(bool on) = 0;
+    // replay the apply from a HIP graph: 0 never, else where it holds few
+    // enough launches
+    virtual void set_graphs(int mode) = 0;
 };
 
 // Host factor (no device needed).
@@ -103,7 +104,7 @@ class IldlPrecond {
     int storage_order = 1;
     int xcd_remap = 1;
     int sell_sigma = 256;  // SELL-C-sigma sorting window of the sweep copies
-    bool graphs = false;   // replay the apply from captured HIP graphs
+    int graphs = -1;       // replay the apply from a HIP graph (0: never)
     // work vectors of an FP32 factor's apply: -1 FP32 for a definite
     // problem and FP64 otherwise, 0 always FP64, 1 always FP32
     int vec32 = -1;

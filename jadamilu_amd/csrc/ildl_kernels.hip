@@ -16,6 +16,9 @@
 
 #include <algorithm>
 #include <climits>
+#include <stdexcept>
+#include <string>
+#include <tuple>
 #include <vector>
 
 namespace jdhip {
@@ -25,6 +28,34 @@ static constexpr int kLpr = 4;
 
 // With xcd != 0 the kernels below take their block id from logical_block()
 // (xcd.hpp): every XCD works on one contiguous range of rows or slices.
+
+// Launch k on q's stream, or add it to q's graph behind the last node.
+template <typename... P, typename... A>
+static void put(const Put &q, void (*k)(P...), int grid, A... args) {
+    if (!q.graph) {
+        k<<<grid, kB, 0, q.stream>>>(args...);
+        return;
+    }
+    std::tuple<P...> held(static_cast<P>(args)...);
+    std::apply(
+        [&](auto &...x) {
+            void *ptrs[] = {(void *)&x...};
+            hipKernelNodeParams np{};
+            np.func = (void *)k;
+            np.gridDim = dim3(grid);
+            np.blockDim = dim3(kB);
+            np.kernelParams = ptrs;
+            hipGraphNode_t node;
+            const hipError_t e =
+                hipGraphAddKernelNode(&node, q.graph, q.last ? &q.last : nullptr,
+                                      q.last ? 1 : 0, &np);
+            if (e != hipSuccess)
+                throw std::runtime_error(std::string("HIP error ") + hipGetErrorString(e) +
+                                         " adding a graph node");
+            q.last = node;
+        },
+        held);
+}
 
 static inline int blocks_for(long n, int per_block, int cap = 8192) {
     long b = (n + per_block - 1) / per_block;
@@ -318,6 +349,11 @@ __global__ __launch_bounds__(kB) void k_zero(int n, W *x) {
         x[i] = W(0);
 }
 template <typename W>
+__global__ __launch_bounds__(kB) void k_copy(int n, const W *__restrict__ t, W *__restrict__ y) {
+    for (long i = blockIdx.x * (long)kB + threadIdx.x; i < n; i += (long)gridDim.x * kB)
+        y[i] = t[i];
+}
+template <typename W>
 __global__ __launch_bounds__(kB) void k_add(int n, const W *__restrict__ t, W *__restrict__ y) {
     for (long i = blockIdx.x * (long)kB + threadIdx.x; i < n; i += (long)gridDim.x * kB)
         y[i] = (W)((double)y[i] + (double)t[i]);
@@ -339,45 +375,45 @@ __global__ __launch_bounds__(kB) void k_dense_gemv(int m, const T *__restrict__ 
 }
 
 template <typename TI, typename W>
-void ildl_gather(hipStream_t s, int n, const int *perm, const double *scal, const TI *in,
+void ildl_gather(const Put &s, int n, const int *perm, const double *scal, const TI *in,
                  W *buf) {
     if (n <= 0) return;
-    k_gather<TI, W><<<blocks_for(n, kB), kB, 0, s>>>(n, perm, scal, in, buf);
+    put(s, k_gather<TI, W>, blocks_for(n, kB), n, perm, scal, in, buf);
 }
 template <typename W, typename TO>
-void ildl_scatter(hipStream_t s, int n, int nB, const int *perm, const double *scal,
+void ildl_scatter(const Put &s, int n, int nB, const int *perm, const double *scal,
                   const W *buf, const W *zc, TO *out) {
     if (n <= 0) return;
-    k_scatter<W, TO><<<blocks_for(n, kB), kB, 0, s>>>(n, nB, perm, scal, buf, zc, out);
+    put(s, k_scatter<W, TO>, blocks_for(n, kB), n, nB, perm, scal, buf, zc, out);
 }
 template <typename T, typename W>
-void ildl_trsv_level(hipStream_t s, const int *rows, int count, const int *ptr, const int *idx,
+void ildl_trsv_level(const Put &s, const int *rows, int count, const int *ptr, const int *idx,
                      const T *val, W *x) {
     if (count <= 0) return;
-    k_trsv_level<T, W><<<blocks_for(count, kB / kLpr), kB, 0, s>>>(rows, count, ptr, idx, val,
+    put(s, k_trsv_level<T, W>, blocks_for(count, kB / kLpr), rows, count, ptr, idx, val,
                                                                    x);
 }
 template <typename T, typename W>
-void ildl_jacobi_sweep_sell(hipStream_t s, const SellView &M, const T *val, const W *b,
+void ildl_jacobi_sweep_sell(const Put &s, const SellView &M, const T *val, const W *b,
                             const W *xin, W *xout, int xcd) {
     if (M.nslices <= 0) return;
     const int g = blocks_for(M.nslices, kB / 64, 1 << 20);
     if (xcd & 2)
-        k_jacobi_sell<T, W, true><<<g, kB, 0, s>>>(M, val, b, xin, xout, xcd & 1);
+        put(s, k_jacobi_sell<T, W, true>, g, M, val, b, xin, xout, xcd & 1);
     else
-        k_jacobi_sell<T, W, false><<<g, kB, 0, s>>>(M, val, b, xin, xout, xcd & 1);
+        put(s, k_jacobi_sell<T, W, false>, g, M, val, b, xin, xout, xcd & 1);
 }
 template <typename T, typename W>
-void ildl_sub_sell(hipStream_t s, const SellView &M, const T *val, const W *x, W *y, int xcd) {
+void ildl_sub_sell(const Put &s, const SellView &M, const T *val, const W *x, W *y, int xcd) {
     if (M.nslices <= 0) return;
-    k_sub_sell<T, W><<<blocks_for(M.nslices, kB / 64, 1 << 20), kB, 0, s>>>(M, val, x, y, xcd);
+    put(s, k_sub_sell<T, W>, blocks_for(M.nslices, kB / 64, 1 << 20), M, val, x, y, xcd);
 }
 template <typename T, typename W>
-void ildl_jacobi_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *idx,
+void ildl_jacobi_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
                      const T *val, const W *b, const W *xin, W *xout, int xcd) {
     if (nrows <= 0) return;
 #define JDHIP_JC(L)                                                                     \
-    k_jacobi_csr<T, W, L><<<blocks_for(nrows, kB / L, 1 << 20), kB, 0, s>>>(nrows, ptr, idx, \
+    put(s, k_jacobi_csr<T, W, L>, blocks_for(nrows, kB / L, 1 << 20), nrows, ptr, idx, \
                                                                             val, b, xin, xout, xcd)
     if (lpr >= 64) JDHIP_JC(64);
     else if (lpr >= 32) JDHIP_JC(32);
@@ -387,11 +423,11 @@ void ildl_jacobi_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const in
 #undef JDHIP_JC
 }
 template <typename T, typename W>
-void ildl_sub_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *idx,
+void ildl_sub_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
                   const T *val, const W *x, W *y, int xcd) {
     if (nrows <= 0) return;
 #define JDHIP_SC(L)                                                                      \
-    k_sub_csr<T, W, L><<<blocks_for(nrows, kB / L, 1 << 20), kB, 0, s>>>(nrows, ptr, idx, val, \
+    put(s, k_sub_csr<T, W, L>, blocks_for(nrows, kB / L, 1 << 20), nrows, ptr, idx, val, \
                                                                          x, y, xcd)
     if (lpr >= 64) JDHIP_SC(64);
     else if (lpr >= 32) JDHIP_SC(32);
@@ -401,13 +437,13 @@ void ildl_sub_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *
 #undef JDHIP_SC
 }
 template <typename T, typename W>
-void ildl_stream(hipStream_t s, const StreamView &M, const int *idx, const T *val, const W *x,
+void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
                  const W *src, W *out, int xcd) {
     if (M.nblk <= 0) return;
     if (M.cap == 512)
-        k_stream<512, T, W><<<M.nblk, kB, 0, s>>>(M, idx, val, x, src, out, xcd);
+        put(s, k_stream<512, T, W>, M.nblk, M, idx, val, x, src, out, xcd);
     else
-        k_stream<1024, T, W><<<M.nblk, kB, 0, s>>>(M, idx, val, x, src, out, xcd);
+        put(s, k_stream<1024, T, W>, M.nblk, M, idx, val, x, src, out, xcd);
 }
 
 // Entries a block holds: 1024 where that leaves enough blocks for the 256 CUs,
@@ -446,63 +482,70 @@ StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vecto
 }
 
 template <typename W>
-void ildl_dscale(hipStream_t s, int n, const double *dinv, W *x) {
+void ildl_dscale(const Put &s, int n, const double *dinv, W *x) {
     if (n <= 0) return;
-    k_dscale<W><<<blocks_for(n, kB), kB, 0, s>>>(n, dinv, x);
+    put(s, k_dscale<W>, blocks_for(n, kB), n, dinv, x);
 }
 template <typename W>
-void ildl_dscale2(hipStream_t s, int n, const double *dinv, const double *doff, const int *pair,
+void ildl_dscale2(const Put &s, int n, const double *dinv, const double *doff, const int *pair,
                   W *x) {
     if (n <= 0) return;
-    k_dscale2<W><<<blocks_for(n, kB), kB, 0, s>>>(n, dinv, doff, pair, x);
+    put(s, k_dscale2<W>, blocks_for(n, kB), n, dinv, doff, pair, x);
 }
-template void ildl_dscale2<double>(hipStream_t, int, const double *, const double *, const int *,
+template void ildl_dscale2<double>(const Put &, int, const double *, const double *, const int *,
                                    double *);
-template void ildl_dscale2<float>(hipStream_t, int, const double *, const double *, const int *,
+template void ildl_dscale2<float>(const Put &, int, const double *, const double *, const int *,
                                   float *);
 template <typename W>
-void ildl_zero(hipStream_t s, int n, W *x) {
+void ildl_zero(const Put &s, int n, W *x) {
     if (n <= 0) return;
-    k_zero<W><<<blocks_for(n, kB), kB, 0, s>>>(n, x);
+    put(s, k_zero<W>, blocks_for(n, kB), n, x);
 }
 template <typename W>
-void ildl_add(hipStream_t s, int n, const W *t, W *y) {
+void ildl_copy(const Put &s, int n, const W *t, W *y) {
     if (n <= 0) return;
-    k_add<W><<<blocks_for(n, kB), kB, 0, s>>>(n, t, y);
+    put(s, k_copy<W>, blocks_for(n, kB), n, t, y);
 }
-template void ildl_zero<double>(hipStream_t, int, double *);
-template void ildl_zero<float>(hipStream_t, int, float *);
-template void ildl_add<double>(hipStream_t, int, const double *, double *);
-template void ildl_add<float>(hipStream_t, int, const float *, float *);
+template void ildl_copy<double>(const Put &, int, const double *, double *);
+template void ildl_copy<float>(const Put &, int, const float *, float *);
+template <typename W>
+void ildl_add(const Put &s, int n, const W *t, W *y) {
+    if (n <= 0) return;
+    put(s, k_add<W>, blocks_for(n, kB), n, t, y);
+}
+template void ildl_zero<double>(const Put &, int, double *);
+template void ildl_zero<float>(const Put &, int, float *);
+template void ildl_add<double>(const Put &, int, const double *, double *);
+template void ildl_add<float>(const Put &, int, const float *, float *);
 template <typename T, typename W>
-void ildl_dense_gemv(hipStream_t s, int m, const T *Minv, const W *x, W *y) {
+void ildl_dense_gemv(const Put &s, int m, const T *Minv, const W *x, W *y) {
     if (m <= 0) return;
-    k_dense_gemv<T, W><<<blocks_for(m, kB / 64, 4096), kB, 0, s>>>(m, Minv, x, y);
+    put(s, k_dense_gemv<T, W>, blocks_for(m, kB / 64, 4096), m, Minv, x, y);
 }
 
 #define INST(T, W)                                                                           \
-    template void ildl_trsv_level<T, W>(hipStream_t, const int *, int, const int *,          \
+    template void ildl_trsv_level<T, W>(const Put &, const int *, int, const int *,          \
                                         const int *, const T *, W *);                        \
-    template void ildl_jacobi_sweep_sell<T, W>(hipStream_t, const SellView &, const T *,      \
+    template void ildl_jacobi_sweep_sell<T, W>(const Put &, const SellView &, const T *,      \
                                                const W *, const W *, W *, int);              \
-    template void ildl_sub_sell<T, W>(hipStream_t, const SellView &, const T *, const W *,    \
+    template void ildl_sub_sell<T, W>(const Put &, const SellView &, const T *, const W *,    \
                                       W *, int);                                             \
-    template void ildl_jacobi_csr<T, W>(hipStream_t, int, int, const int *, const int *,      \
+    template void ildl_jacobi_csr<T, W>(const Put &, int, int, const int *, const int *,      \
                                         const T *, const W *, const W *, W *, int);          \
-    template void ildl_sub_csr<T, W>(hipStream_t, int, int, const int *, const int *,         \
+    template void ildl_sub_csr<T, W>(const Put &, int, int, const int *, const int *,         \
                                      const T *, const W *, W *, int);                        \
-    template void ildl_dense_gemv<T, W>(hipStream_t, int, const T *, const W *, W *);         \
-    template void ildl_stream<T, W>(hipStream_t, const StreamView &, const int *, const T *,   \
+    template void ildl_dense_gemv<T, W>(const Put &, int, const T *, const W *, W *);         \
+    template void ildl_stream<T, W>(const Put &, const StreamView &, const int *, const T *,   \
                                     const W *, const W *, W *, int);
 INST(double, double)
 INST(float, double)
 INST(float, float)
-template void ildl_dscale<double>(hipStream_t, int, const double *, double *);
-template void ildl_dscale<float>(hipStream_t, int, const double *, float *);
+template void ildl_dscale<double>(const Put &, int, const double *, double *);
+template void ildl_dscale<float>(const Put &, int, const double *, float *);
 #define INST_IO(A, B)                                                                        \
-    template void ildl_gather<A, B>(hipStream_t, int, const int *, const double *, const A *, \
+    template void ildl_gather<A, B>(const Put &, int, const int *, const double *, const A *, \
                                     B *);                                                    \
-    template void ildl_scatter<B, A>(hipStream_t, int, int, const int *, const double *,      \
+    template void ildl_scatter<B, A>(const Put &, int, int, const int *, const double *,      \
                                      const B *, const B *, A *);
 INST_IO(double, double)
 INST_IO(double, float)

@@ -19,17 +19,29 @@
 
 namespace jdhip {
 
+// Where the launches below go: onto a stream or, when graph is set, behind the
+// last node of a graph that is being built.  The graph is built node by node
+// and not by capture: a capture would make other threads' work on the legacy
+// null stream fail while it lasts.
+struct Put {
+    hipStream_t stream = nullptr;
+    hipGraph_t graph = nullptr;
+    mutable hipGraphNode_t last = nullptr;
+    Put(hipStream_t s) : stream(s) {}
+    Put(hipGraph_t g) : graph(g) {}
+};
+
 // Factor values are T (double or float), work vectors W (double or float);
 // sums are double.
 template <typename TI, typename W>
-void ildl_gather(hipStream_t s, int n, const int *perm, const double *scal, const TI *in,
+void ildl_gather(const Put &s, int n, const int *perm, const double *scal, const TI *in,
                  W *buf);
 template <typename W, typename TO>
-void ildl_scatter(hipStream_t s, int n, int nB, const int *perm, const double *scal,
+void ildl_scatter(const Put &s, int n, int nB, const int *perm, const double *scal,
                   const W *buf, const W *zc, TO *out);
 // x[rows of one level] -= sum_j M(row, j) x[j]   (unit-diagonal triangular)
 template <typename T, typename W>
-void ildl_trsv_level(hipStream_t s, const int *rows, int count, const int *ptr, const int *idx,
+void ildl_trsv_level(const Put &s, const int *rows, int count, const int *ptr, const int *idx,
                      const T *val, W *x);
 // Device view of a SELL-C-sigma matrix: slices of 64 rows (one wave64, one
 // lane per row) taken from windows of rows sorted by length; entries of a
@@ -50,19 +62,19 @@ struct SellView {
 // One Jacobi sweep of the unit triangle, xout = b - M xin.  xcd bit 0:
 // XCD-contiguous block order; bit 1: nontemporal loads of the matrix stream.
 template <typename T, typename W>
-void ildl_jacobi_sweep_sell(hipStream_t s, const SellView &M, const T *val, const W *b,
+void ildl_jacobi_sweep_sell(const Put &s, const SellView &M, const T *val, const W *b,
                             const W *xin, W *xout, int xcd);
 // CSR forms with lpr (4, 8, 16, 32 or 64) lanes per row, for matrices with long rows;
 // xcd != 0: XCD-contiguous block order (as for the SELL and stream forms)
 template <typename T, typename W>
-void ildl_jacobi_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *idx,
+void ildl_jacobi_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
                      const T *val, const W *b, const W *xin, W *xout, int xcd);
 template <typename T, typename W>
-void ildl_sub_csr(hipStream_t s, int lpr, int nrows, const int *ptr, const int *idx,
+void ildl_sub_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
                   const T *val, const W *x, W *y, int xcd);
 // y[r] -= sum_j M(r, j) x[j] over the rows of a SELL-C-sigma matrix
 template <typename T, typename W>
-void ildl_sub_sell(hipStream_t s, const SellView &M, const T *val, const W *x, W *y, int xcd);
+void ildl_sub_sell(const Put &s, const SellView &M, const T *val, const W *x, W *y, int xcd);
 // CSR-stream form: blocks of consecutive rows with at most cap - 2 entries
 // (and 256 rows) each, or one longer row, streamed through LDS with coalesced
 // loads.  The product reads the CSR's own values and columns (which end in
@@ -89,24 +101,27 @@ StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vecto
 // out = src - M x over every row (a sweep: src = b; a product: src = out = y).
 // xcd != 0: every XCD takes one contiguous range of row blocks.
 template <typename T, typename W>
-void ildl_stream(hipStream_t s, const StreamView &M, const int *idx, const T *val, const W *x,
+void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
                  const W *src, W *out, int xcd);
 template <typename W>
-void ildl_dscale(hipStream_t s, int n, const double *dinv, W *x);
+void ildl_dscale(const Put &s, int n, const double *dinv, W *x);
 // x = D^-1 x with 2x2 blocks: row i pairs with pair[i] (-1: 1x1 pivot,
 // x_i *= dinv_i); a pair is updated by its lower index,
 // (x_i, x_p) <- (dinv_i x_i + doff_i x_p, doff_p x_i + dinv_p x_p)
 template <typename W>
-void ildl_dscale2(hipStream_t s, int n, const double *dinv, const double *doff, const int *pair,
+void ildl_dscale2(const Put &s, int n, const double *dinv, const double *doff, const int *pair,
                   W *x);
 // x = 0 (a kernel, not a memset: the apply may be captured in a HIP graph)
 template <typename W>
-void ildl_zero(hipStream_t s, int n, W *x);
+void ildl_zero(const Put &s, int n, W *x);
+// y = t
+template <typename W>
+void ildl_copy(const Put &s, int n, const W *t, W *y);
 // y += t
 template <typename W>
-void ildl_add(hipStream_t s, int n, const W *t, W *y);
+void ildl_add(const Put &s, int n, const W *t, W *y);
 // y = Minv x, Minv m x m row-major
 template <typename T, typename W>
-void ildl_dense_gemv(hipStream_t s, int m, const T *Minv, const W *x, W *y);
+void ildl_dense_gemv(const Put &s, int m, const T *Minv, const W *x, W *y);
 
 }  // namespace jdhip

@@ -64,3 +64,34 @@ def test_stream_rows_at_the_block_size(k, single):
 # a level large enough for the blocks of 1022 entries
 def test_stream_wide_blocks():
     _check(lambda: M.laplace((64, 63, 61)), {"ildl_form": 1}, 2)
+
+
+def test_apply_on_a_stream_under_capture():
+    """A replayed apply launches kernel by kernel while its stream is captured
+    (a graph launch cannot be), and the captured graph gives the same values
+    on every replay, with the context's own replays between them."""
+    from jadamilu_amd.ildl import IldlFactor
+    from jadamilu_amd.jd import Context
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    ia, ja, a = M.laplace((20, 19, 18))
+    n = ia.size - 1
+    ctx = Context(0)
+    ctx.attach_ildl(IldlFactor(n, ia, ja, a, droptol=1e-3, spd=True, dense_max=100), sweeps=3)
+    r = torch.rand(n, dtype=torch.float64, device="cuda:0")
+    z, zc = torch.zeros_like(r), torch.zeros_like(r)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.ExternalStream(ctx.stream_ptr()),
+                          capture_error_mode="thread_local"):
+        ctx.precond_apply(zc.data_ptr(), r.data_ptr())
+    for _ in range(4):
+        r.uniform_(-1.0, 1.0)
+        zc.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        ctx.precond_apply(z.data_ptr(), r.data_ptr())
+        torch.cuda.synchronize()
+        assert torch.equal(z, zc) and float(z.abs().max()) > 0.0
+    ctx.close()
