@@ -687,7 +687,7 @@ def main():
         sw_ms, sw_bytes = ctx.ildl_time_sweep(args.spmv_reps)
         sw_ach = sw_bytes / (sw_ms * 1e-3) / 1e9
         form = pinfo["level_forms"][0][0] if pinfo and pinfo.get("level_forms") else 0
-        kname = {0: "k_jacobi_sell", 1: "k_stream"}.get(form, f"k_jacobi_csr<{form}>")
+        kname = {0: "k_sell", 1: "k_stream"}.get(form, f"k_csr<{form}>")
         kdesc = {0: "SELL-C-sigma, one lane per row",
                  1: "CSR-stream, row blocks through LDS"}.get(form, f"CSR, {form} lanes per row")
         # the traffic file holds counters of one kernel form; use them only

@@ -206,15 +206,19 @@ struct SellDev {
     long nnz16 = 0, nnz32 = 0;
 };
 
-// Lanes per row for a product with nnz entries over rows rows: one lane per
-// row (SELL) for short rows, CSR lane groups for long rows or small levels.
-inline int pick_lanes(long nnz, int rows) {
+// Kernel form of a product with nnz entries over rows rows before any timing:
+// CSR-stream for large products, whose entries it balances, else CSR lane
+// groups of about the average row length.  Measured (us a launch in a graph,
+// stream / the rule's lanes): 609k entries of 22 a row 5.4 / 6.2, 354k of 98
+// 3.8 / 3.9, 186k of 16 3.5 / 3.3, 107k of 134 3.8 / 3.1, 22k of 2.8 3.2 / 2.6.
+constexpr long kTimed = 200000;
+inline int pick_form(long nnz, int rows) {
     if (rows <= 0) return 0;
-    const double avg = (double)nnz / rows;
-    if (avg >= 96.0) return 64;
-    if (avg >= 24.0) return 16;
-    if (rows < 65536 && avg >= 6.0) return 4;
-    return 0;
+    if (nnz >= kTimed || rows >= 32768) return 1;
+    const double avg = 0.8 * (double)nnz / rows;
+    int lanes = 8;
+    while (lanes < 64 && lanes < avg) lanes *= 2;
+    return lanes;
 }
 
 template <typename T, typename W>
@@ -385,15 +389,15 @@ class IldlImpl : public IldlImplBase {
             D.lc_idx = track(dev_upload(ctx_->stream, ci, kStreamPad));
             D.lc_val = track(dev_upload(ctx_->stream, cv, kStreamPad));
             D.st_c = upload_stream(nC, cp, ci);
-            D.wc = pick_lanes((long)ci.size(), nC);
-            D.wf = D.wb = pick_lanes((long)bi.size(), nB);
+            D.wc = pick_form((long)ci.size(), nC);
+            D.wf = D.wb = pick_form((long)bi.size(), nB);
             transpose(nC, nB, cp, ci, cv, tp, ti, tv);
             D.sct = upload_sell(build_sell(nB, tp, ti, tv, sigma_, true));
             D.lct_ptr = track(dev_upload(ctx_->stream, tp));
             D.lct_idx = track(dev_upload(ctx_->stream, ti, kStreamPad));
             D.lct_val = track(dev_upload(ctx_->stream, tv, kStreamPad));
             D.st_ct = upload_stream(nB, tp, ti);
-            D.wct = pick_lanes((long)ti.size(), nB);
+            D.wct = pick_form((long)ti.size(), nB);
             D.buf = track(dev_alloc<W>(n));
             D.out = track(dev_alloc<W>(n));
             D.t1 = track(dev_alloc<W>(std::max(nB, 1)));
@@ -430,99 +434,124 @@ class IldlImpl : public IldlImplBase {
         JDHIP_CHECK(hipStreamSynchronize(ctx_->stream));
     }
 
-    // Triangular solve with L_B (fwd) or L_B^T in place on x (nB entries).
-    void tri_solve(const Put &s, const DevLevel<T, W> &D, bool fwd, W *x) {
-        const int *ptr = fwd ? D.lb_ptr : D.lt_ptr;
-        const int *idx = fwd ? D.lb_idx : D.lt_idx;
-        const T *val = fwd ? D.lb_val : D.lt_val;
+    // Triangular solve with L_B (fwd) or L_B^T on x (nB entries), then times
+    // dinv and added to add (both may be null, see RowOp), into out (which may
+    // be x, and add).
+    void tri_solve(const Put &s, const DevLevel<T, W> &D, bool fwd, W *x, const double *dinv,
+                   const W *add, W *out) {
         const int nsw = D.k;
         if (nsw <= 0) {
+            const int *ptr = fwd ? D.lb_ptr : D.lt_ptr;
+            const int *idx = fwd ? D.lb_idx : D.lt_idx;
+            const T *val = fwd ? D.lb_val : D.lt_val;
             const std::vector<int> &lp = fwd ? D.fwd_ptr : D.bwd_ptr;
             const int *rows = fwd ? D.fwd_rows : D.bwd_rows;
             for (size_t l = 1; l + 1 < lp.size(); ++l)  // level 0 rows have no entries
                 ildl_trsv_level<T, W>(s, rows + lp[l], lp[l + 1] - lp[l], ptr, idx, val, x);
+            if (dinv) ildl_dscale<W>(s, D.nB, dinv, x);
+            if (add) ildl_add<W>(s, D.nB, x, out);
             return;
         }
         // Jacobi sweeps y <- b - N y from y = b (b = x).  The first sweep
-        // reads b itself; the last writes into x, which is safe because
-        // every row reads only its own b entry and all y entries come from
-        // the other buffer (needs at least 2 sweeps; 1 sweep goes via t1).
-        const int lanes = fwd ? D.wf : D.wb;
-        const W *xin = x;
+        // reads b itself; the last writes out, which may be x: every row
+        // reads only its own b entry and all y entries come from the other
+        // buffer (a single sweep into x goes via t1).
         W *bufs[2] = {D.t1, D.t2};
+        const W *xin = x;
         for (int k = 0; k < nsw; ++k) {
-            const bool last = (k == nsw - 1) && nsw >= 2;
-            W *xout = last ? x : bufs[k & 1];
-            sweep_launch(s, D, fwd, lanes, x, xin, xout);
-            xin = xout;
+            RowOp<W> op;
+            op.src = x;
+            op.out = bufs[k & 1];
+            if (k == nsw - 1) {
+                op.dinv = dinv;
+                op.add = add;
+                if (out != xin) op.out = out;
+            }
+            sweep_launch(s, D, fwd, fwd ? D.wf : D.wb, xin, op);
+            xin = op.out;
         }
-        if (nsw == 1) ildl_copy<W>(s, D.nB, D.t1, x);
+        if (xin != out) ildl_copy<W>(s, D.nB, xin, out);
     }
 
-    // One Jacobi sweep xout = b - N xin of the level's L_B (fwd) or L_B^T,
-    // in the given kernel form: 0 one lane per row on the SELL-C-sigma copy,
-    // else CSR with that many lanes per row.
-    void sweep_launch(const Put &s, const DevLevel<T, W> &D, bool fwd, int form, const W *b,
-                      const W *xin, W *xout) {
+    // One product with the level's L_B (fwd) or L_B^T in the given kernel
+    // form: 0 one lane per row on the SELL-C-sigma copy, 1 CSR-stream, else
+    // CSR with that many lanes per row.
+    void sweep_launch(const Put &s, const DevLevel<T, W> &D, bool fwd, int form, const W *x,
+                      const RowOp<W> &op) {
+        const int *idx = fwd ? D.lb_idx : D.lt_idx;
+        const T *val = fwd ? D.lb_val : D.lt_val;
         if (form == 1) {
-            ildl_stream<T, W>(s, fwd ? D.st_b : D.st_t, fwd ? D.lb_idx : D.lt_idx,
-                              fwd ? D.lb_val : D.lt_val, xin, b, xout, xcd_ & 1);
+            ildl_stream<T, W>(s, fwd ? D.st_b : D.st_t, idx, val, x, op, xcd_ & 1);
         } else if (form > 0) {
-            ildl_jacobi_csr<T, W>(s, form, D.nB, fwd ? D.lb_ptr : D.lt_ptr,
-                                  fwd ? D.lb_idx : D.lt_idx, fwd ? D.lb_val : D.lt_val, b, xin,
-                                  xout, xcd_ & 1);
+            ildl_csr<T, W>(s, form, D.nB, fwd ? D.lb_ptr : D.lt_ptr, idx, val, x, op, xcd_ & 1);
         } else {
             const SellDev<T> &M = fwd ? D.sf : D.sb;
-            ildl_jacobi_sweep_sell<T, W>(s, M.v, M.val, b, xin, xout, xcd_);
+            ildl_sell<T, W>(s, M.v, M.val, x, op, xcd_);
         }
     }
-    // y -= L_CB x (C rows; trans = false) or y -= L_CB^T x (B rows)
+    // y -= L_CB x (C rows; trans = false) or y -= L_CB^T x (B rows); with
+    // fresh, y = -(the product)
     void sub_launch(const Put &s, const DevLevel<T, W> &D, bool trans, int form, const W *x,
-                    W *y) {
+                    W *y, bool fresh = false) {
+        const int rows = trans ? D.nB : D.nC;
+        const int *idx = trans ? D.lct_idx : D.lc_idx;
+        const T *val = trans ? D.lct_val : D.lc_val;
+        RowOp<W> op;
+        op.src = fresh ? nullptr : y;
+        op.out = y;
         if (form == 1) {
-            ildl_stream<T, W>(s, trans ? D.st_ct : D.st_c, trans ? D.lct_idx : D.lc_idx,
-                              trans ? D.lct_val : D.lc_val, x, y, y, xcd_ & 1);
+            ildl_stream<T, W>(s, trans ? D.st_ct : D.st_c, idx, val, x, op, xcd_ & 1);
         } else if (form > 0) {
-            if (trans)
-                ildl_sub_csr<T, W>(s, form, D.nB, D.lct_ptr, D.lct_idx, D.lct_val, x, y,
-                                   xcd_ & 1);
-            else
-                ildl_sub_csr<T, W>(s, form, D.nC, D.lc_ptr, D.lc_idx, D.lc_val, x, y,
-                                   xcd_ & 1);
+            ildl_csr<T, W>(s, form, rows, trans ? D.lct_ptr : D.lc_ptr, idx, val, x, op,
+                           xcd_ & 1);
         } else {
+            // this copy has no lanes for empty rows
+            if (fresh) ildl_zero<W>(s, rows, y);
+            op.src = y;
             const SellDev<T> &M = trans ? D.sct : D.sc;
-            ildl_sub_sell<T, W>(s, M.v, M.val, x, y, xcd_);
+            ildl_sell<T, W>(s, M.v, M.val, x, op, xcd_ & 1);
         }
     }
 
     // Kernel form of every product of every level (both sweeps, L_CB and
-    // L_CB^T) by measurement: the fastest of one lane per row on the
-    // SELL-C-sigma copy, the CSR-stream form (form 1) and CSR with 4, 8, 16,
-    // 32 or 64 lanes per row, each timed
-    // over three launches on zeroed vectors.  Replaces the row-length
-    // heuristic the upload starts from.
+    // L_CB^T).  Products of at least kTimed entries by measurement: the fastest
+    // of one lane per row on the SELL-C-sigma copy, the CSR-stream form (form
+    // 1) and CSR with 4 to 64 lanes per row, each timed over six launches of a
+    // graph on zeroed vectors (launched one by one they would be timed at the
+    // host's rate).  Smaller ones differ by less than a timing is worth and
+    // keep the lanes of the upload's rule.
     void autotune_forms() override {
         hipStream_t s = ctx_->stream;
         hipEvent_t e0, e1;
         JDHIP_CHECK(hipEventCreate(&e0));
         JDHIP_CHECK(hipEventCreate(&e1));
         auto timed = [&](auto &&launch) {
-            launch();
-            JDHIP_CHECK(hipEventRecord(e0, s));
-            for (int i = 0; i < 3; ++i) launch();
-            JDHIP_CHECK(hipEventRecord(e1, s));
-            JDHIP_CHECK(hipEventSynchronize(e1));
-            float ms = 0.f;
-            JDHIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-            return ms;
+            hipGraph_t g = nullptr;
+            hipGraphExec_t x = nullptr;
+            JDHIP_CHECK(hipGraphCreate(&g, 0));
+            const Put q(g);
+            for (int i = 0; i < 6; ++i) launch(q);
+            JDHIP_CHECK(hipGraphInstantiate(&x, g, nullptr, nullptr, 0));
+            JDHIP_CHECK(hipGraphDestroy(g));
+            float best = 0.f;
+            for (int i = 0; i < 3; ++i) {
+                JDHIP_CHECK(hipEventRecord(e0, s));
+                JDHIP_CHECK(hipGraphLaunch(x, s));
+                JDHIP_CHECK(hipEventRecord(e1, s));
+                JDHIP_CHECK(hipEventSynchronize(e1));
+                float ms = 0.f;
+                JDHIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+                if (i == 1 || ms < best) best = ms;  // the first one warms up
+            }
+            JDHIP_CHECK(hipGraphExecDestroy(x));
+            return best;
         };
-        const int forms[7] = {0, 1, 4, 8, 16, 32, 64};
         auto best = [&](auto &&launch_form) {
-            int bf = 0;
+            int bf = 1;
             float bt = 0.f;
-            for (int f : forms) {
-                const float t = timed([&] { launch_form(f); });
-                if (f == 0 || t < bt) {
+            for (int f : {1, 0, 4, 8, 16, 32, 64}) {
+                const float t = timed([&](const Put &q) { launch_form(q, f); });
+                if (f == 1 || t < bt) {
                     bt = t;
                     bf = f;
                 }
@@ -530,17 +559,25 @@ class IldlImpl : public IldlImplBase {
             return bf;
         };
         for (auto &D : lv_) {
-            JDHIP_CHECK(hipMemsetAsync(D.buf, 0, sizeof(W) * D.n, s));
-            JDHIP_CHECK(hipMemsetAsync(D.out, 0, sizeof(W) * D.n, s));
-            JDHIP_CHECK(hipMemsetAsync(D.t1, 0, sizeof(W) * std::max(D.nB, 1), s));
-            JDHIP_CHECK(hipMemsetAsync(D.t2, 0, sizeof(W) * std::max(D.nB, 1), s));
-            if (D.nB > 0) {
-                D.wf = best([&](int f) { sweep_launch(s, D, true, f, D.buf, D.t1, D.t2); });
-                D.wb = best([&](int f) { sweep_launch(s, D, false, f, D.buf, D.t1, D.t2); });
+            if (D.nnz_lb < kTimed && D.nnz_lc < kTimed) continue;
+            ildl_zero<W>(s, D.n, D.buf);
+            ildl_zero<W>(s, D.n, D.out);
+            ildl_zero<W>(s, D.nB, D.t1);
+            ildl_zero<W>(s, D.nB, D.t2);
+            RowOp<W> op;
+            op.src = D.buf;
+            op.out = D.t2;
+            if (D.nB > 0 && D.nnz_lb >= kTimed) {
+                D.wf = best([&](const Put &q, int f) { sweep_launch(q, D, true, f, D.t1, op); });
+                D.wb = best([&](const Put &q, int f) { sweep_launch(q, D, false, f, D.t1, op); });
             }
-            if (D.nC > 0) {
-                D.wc = best([&](int f) { sub_launch(s, D, false, f, D.buf, D.buf + D.nB); });
-                D.wct = best([&](int f) { sub_launch(s, D, true, f, D.out, D.buf); });
+            if (D.nC > 0 && D.nnz_lc >= kTimed) {
+                D.wc = best([&](const Put &q, int f) {
+                    sub_launch(q, D, false, f, D.buf, D.buf + D.nB);
+                });
+                D.wct = best([&](const Put &q, int f) {
+                    sub_launch(q, D, true, f, D.out, D.buf, fform());
+                });
             }
         }
         JDHIP_CHECK(hipStreamSynchronize(s));
@@ -791,15 +828,15 @@ class IldlImpl : public IldlImplBase {
                 const DevLevel<T, W> &P = lv_[l - 1];
                 ildl_gather<W, W>(s, D.n, D.perm, D.scal, P.buf + P.nB, D.buf);
             }
-            tri_solve(s, D, true, D.buf);
             if (fform()) {
                 // y_B = B^-1 b_B, then b_C -= F^T y_B
-                dscale(s, D, D.buf);
-                tri_solve(s, D, false, D.buf);
+                block_solve(s, D, D.buf, nullptr, D.buf);
                 if (D.nC > 0) sub_launch(s, D, false, D.wc, D.buf, D.buf + D.nB);
             } else {
+                tri_solve(s, D, true, D.buf, nullptr, nullptr, D.buf);
                 if (D.nC > 0) sub_launch(s, D, false, D.wc, D.buf, D.buf + D.nB);
-                dscale(s, D, D.buf);
+                if (!D.dpair) ildl_dscale<W>(s, D.nB, D.dinv, D.buf);
+                else ildl_dscale2<W>(s, D.nB, D.dinv, D.doinv, D.dpair, D.buf);
             }
         }
         if (f_.m > 0) {
@@ -813,26 +850,25 @@ class IldlImpl : public IldlImplBase {
                 if (D.nC > 0) {
                     // x_B = y_B - B^-1 F x_C; D.out is free until the scatter
                     W *t = D.out;
-                    ildl_zero<W>(s, D.nB, t);
-                    sub_launch(s, D, true, D.wct, zc, t);
-                    tri_solve(s, D, true, t);
-                    dscale(s, D, t);
-                    tri_solve(s, D, false, t);
-                    ildl_add<W>(s, D.nB, t, D.buf);
+                    sub_launch(s, D, true, D.wct, zc, t, true);
+                    block_solve(s, D, t, D.buf, D.buf);
                 }
             } else {
                 if (D.nC > 0) sub_launch(s, D, true, D.wct, zc, D.buf);
-                tri_solve(s, D, false, D.buf);
+                tri_solve(s, D, false, D.buf, nullptr, nullptr, D.buf);
             }
             if (l > 0) ildl_scatter<W, W>(s, D.n, D.nB, D.perm, D.scal, D.buf, zc, D.out);
         }
     }
 
     bool fform() const { return f_.coupling == 0; }
-    // x_B = D^-1 x_B (1x1 and 2x2 pivots)
-    void dscale(const Put &s, const DevLevel<T, W> &D, W *x) {
+    // out = add + B^-1 x (add may be null): forward solve, D^-1 (1x1 pivots in
+    // the last forward sweep, 2x2 pivots by a launch of their own), backward
+    // solve; x is overwritten
+    void block_solve(const Put &s, const DevLevel<T, W> &D, W *x, const W *add, W *out) {
+        tri_solve(s, D, true, x, D.dpair ? nullptr : D.dinv, nullptr, x);
         if (D.dpair) ildl_dscale2<W>(s, D.nB, D.dinv, D.doinv, D.dpair, x);
-        else ildl_dscale<W>(s, D.nB, D.dinv, x);
+        tri_solve(s, D, false, x, nullptr, add, out);
     }
     int nlevels() const override { return (int)f_.levels.size(); }
     int dense_m() const override { return f_.m; }
@@ -879,7 +915,7 @@ class IldlImpl : public IldlImplBase {
             const long solves = (fform() && D.nC > 0) ? 2 : 1;
             b += solves * (k * (mat_bytes(D.sf, D.wf, D.nnz_lb) + mat_bytes(D.sb, D.wb, D.nnz_lb)) +
                            2 * k * (4L * D.nB + 3 * v * D.nB));
-            if (solves == 2) b += 2 * v * D.nB * 3;  // second D^-1, zero, add
+            if (solves == 2) b += v * D.nB;  // y_B, added to
             b += mat_bytes(D.sc, D.wc, D.nnz_lc) + mat_bytes(D.sct, D.wct, D.nnz_lc) +
                  2 * (4L * (D.nC + D.nB + 2) + v * (D.nB + D.nC));
             b += 2 * (4L + v) * D.n + 2 * v * D.n + 2 * v * D.nB;
@@ -898,7 +934,10 @@ class IldlImpl : public IldlImplBase {
         hipEvent_t e0, e1;
         JDHIP_CHECK(hipEventCreate(&e0));
         JDHIP_CHECK(hipEventCreate(&e1));
-        auto one = [&]() { sweep_launch(s, D, true, D.wf, D.buf, D.t1, D.t2); };
+        RowOp<W> op;
+        op.src = D.buf;
+        op.out = D.t2;
+        auto one = [&]() { sweep_launch(s, D, true, D.wf, D.t1, op); };
         one();
         JDHIP_CHECK(hipEventRecord(e0, s));
         for (int i = 0; i < reps; ++i) one();

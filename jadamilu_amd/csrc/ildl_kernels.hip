@@ -141,33 +141,34 @@ __device__ __forceinline__ double sell_slice_row(const SellView &M, const T *__r
     return sell_row<NT>(v, (const int *)(M.idx + M.iptr[sl]) + lane, 0, code >> 1, x);
 }
 
-template <typename T, typename W, bool NT>
-__global__ __launch_bounds__(kB) void k_jacobi_sell(SellView M, const T *__restrict__ val,
-                                                    const W *b, const W *xin, W *xout,
-                                                    int xcd) {
-    // b and xout may be the same array (the last sweep writes in place: each
-    // lane reads b only at its own row before writing that row)
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (long sl = logical_block(xcd) * (kB / 64) + wv; sl < M.nslices;
-         sl += (long)gridDim.x * (kB / 64)) {
-        const int r = M.rowid[sl * 64 + lane];
-        if (r < 0) continue;
-        const double s = sell_slice_row<NT>(M, val, sl, lane, xin);
-        xout[r] = (W)((double)b[r] - s);
+// One row of a RowOp: its inputs, loaded ahead of the row's sum, and the write.
+template <typename W>
+struct RowIn {
+    double src = 0.0, dinv = 1.0, add = 0.0;
+    __device__ __forceinline__ void load(const RowOp<W> &op, long r) {
+        if (op.src) src = (double)op.src[r];
+        if (op.dinv) dinv = op.dinv[r];
+        if (op.add) add = (double)op.add[r];
     }
-}
+    __device__ __forceinline__ void store(const RowOp<W> &op, long r, double sum) const {
+        W v = (W)(src - sum);
+        if (op.dinv) v = (W)((double)v * dinv);
+        if (op.add) v = (W)(add + (double)v);
+        op.out[r] = v;
+    }
+};
 
-template <typename T, typename W>
-__global__ __launch_bounds__(kB) void k_sub_sell(SellView M, const T *__restrict__ val,
-                                                 const W *__restrict__ x, W *__restrict__ y,
-                                                 int xcd) {
+template <typename T, typename W, bool NT>
+__global__ __launch_bounds__(kB) void k_sell(SellView M, const T *__restrict__ val, const W *x,
+                                             RowOp<W> op, int xcd) {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (long sl = logical_block(xcd) * (kB / 64) + wv; sl < M.nslices;
          sl += (long)gridDim.x * (kB / 64)) {
         const int r = M.rowid[sl * 64 + lane];
         if (r < 0) continue;
-        const double s = sell_slice_row<false>(M, val, sl, lane, x);
-        y[r] = (W)((double)y[r] - s);
+        RowIn<W> in;
+        in.load(op, r);
+        in.store(op, r, sell_slice_row<NT>(M, val, sl, lane, x));
     }
 }
 
@@ -175,35 +176,22 @@ __global__ __launch_bounds__(kB) void k_sub_sell(SellView M, const T *__restrict
 // reduction inside the lane group): with one lane per row such levels keep
 // too few waves in flight and each lane walks its row serially.
 template <typename T, typename W, int LPR>
-__global__ __launch_bounds__(kB) void k_jacobi_csr(int nrows, const int *__restrict__ ptr,
-                                                   const int *__restrict__ idx,
-                                                   const T *__restrict__ val, const W *b,
-                                                   const W *xin, W *xout, int xcd) {
+__global__ __launch_bounds__(kB) void k_csr(int nrows, const int *__restrict__ ptr,
+                                            const int *__restrict__ idx,
+                                            const T *__restrict__ val, const W *x, RowOp<W> op,
+                                            int xcd) {
     const int g = threadIdx.x / LPR, l = threadIdx.x % LPR;
     for (long r = logical_block(xcd) * (kB / LPR) + g; r < nrows; r += (long)gridDim.x * (kB / LPR)) {
-        double s = csr_lane_sum<LPR>(idx, val, xin, ptr[r], ptr[r + 1], l);
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
-        if (l == 0) xout[r] = (W)((double)b[r] - s);
-    }
-}
-
-template <typename T, typename W, int LPR>
-__global__ __launch_bounds__(kB) void k_sub_csr(int nrows, const int *__restrict__ ptr,
-                                                const int *__restrict__ idx,
-                                                const T *__restrict__ val,
-                                                const W *__restrict__ x, W *__restrict__ y,
-                                                int xcd) {
-    const int g = threadIdx.x / LPR, l = threadIdx.x % LPR;
-    for (long r = logical_block(xcd) * (kB / LPR) + g; r < nrows; r += (long)gridDim.x * (kB / LPR)) {
+        RowIn<W> in;
+        if (l == 0) in.load(op, r);
         double s = csr_lane_sum<LPR>(idx, val, x, ptr[r], ptr[r + 1], l);
 #pragma unroll
         for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
-        if (l == 0) y[r] = (W)((double)y[r] - s);
+        if (l == 0) in.store(op, r, s);
     }
 }
 
-// CSR-stream form, out = src - M x: a block owns a run of consecutive rows
+// CSR-stream form: a block owns a run of consecutive rows
 // with at most CAP - 2 entries (and at most kB rows), or a single longer row.
 // It streams the entries of its rows (consecutive in CSR) with coalesced,
 // independent loads, parks the products in LDS, then sums each row with a
@@ -212,7 +200,7 @@ __global__ __launch_bounds__(kB) void k_sub_csr(int nrows, const int *__restrict
 //
 // Bound by memory on large levels and by the chain of dependent loads on
 // small ones, so the chain is kept to three: the block's descriptor; then
-// columns, values, the row's entry range and src together; then the gathers
+// columns, values, the row's entry range and its RowOp inputs together; then the gathers
 // of x.  A thread takes entries in pairs (16 bytes of values, 4 or 8 of
 // columns a load); pairs start at an even entry, so the first may hold an
 // entry of the block before and the last one of the block behind, which are
@@ -225,7 +213,7 @@ __global__ __launch_bounds__(kB) void k_sub_csr(int nrows, const int *__restrict
 template <int CAP, typename T, typename W>
 __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restrict__ idx,
                                                const T *__restrict__ val, const W *x,
-                                               const W *src, W *out, int xcd) {
+                                               RowOp<W> op, int xcd) {
     typedef T T2 __attribute__((ext_vector_type(2)));
     __shared__ __align__(16) double prod[CAP];
     __shared__ double red[kB / 64];
@@ -254,7 +242,9 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restri
             double t = 0.0;
 #pragma unroll
             for (int w = 0; w < kB / 64; ++w) t += red[w];
-            out[r0] = (W)((double)src[r0] - t);
+            RowIn<W> in;
+            in.load(op, r0);
+            in.store(op, r0, t);
         }
         return;
     }
@@ -263,12 +253,12 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restri
     const int g = tid / t, l = tid % t;
     const bool mine = g < nr;
     int a = 0, b = 0;
-    double sv = 0.0;
+    RowIn<W> in;
     if (mine) {
         const unsigned short *o = M.off + (r0 + blk + g);
         a = o[0];
         b = o[1];
-        if (l == 0) sv = (double)src[r0 + g];
+        if (l == 0) in.load(op, r0 + g);
     }
     const int ea = e0 & ~1, sh = e0 & 1, tot = ne + sh;  // entries from the even start on
     if (ne > 0) {
@@ -318,7 +308,7 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restri
     if (mine)
         for (int k = sh + a + l; k < sh + b; k += t) s += prod[k];
     for (int o = t / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, t);
-    if (mine && l == 0) out[r0 + g] = (W)(sv - s);
+    if (mine && l == 0) in.store(op, r0 + g, s);
 }
 
 template <typename W>
@@ -394,56 +384,32 @@ void ildl_trsv_level(const Put &s, const int *rows, int count, const int *ptr, c
                                                                    x);
 }
 template <typename T, typename W>
-void ildl_jacobi_sweep_sell(const Put &s, const SellView &M, const T *val, const W *b,
-                            const W *xin, W *xout, int xcd) {
+void ildl_sell(const Put &s, const SellView &M, const T *val, const W *x, const RowOp<W> &op,
+               int xcd) {
     if (M.nslices <= 0) return;
     const int g = blocks_for(M.nslices, kB / 64, 1 << 20);
-    if (xcd & 2)
-        put(s, k_jacobi_sell<T, W, true>, g, M, val, b, xin, xout, xcd & 1);
-    else
-        put(s, k_jacobi_sell<T, W, false>, g, M, val, b, xin, xout, xcd & 1);
+    if (xcd & 2) put(s, k_sell<T, W, true>, g, M, val, x, op, xcd & 1);
+    else put(s, k_sell<T, W, false>, g, M, val, x, op, xcd & 1);
 }
 template <typename T, typename W>
-void ildl_sub_sell(const Put &s, const SellView &M, const T *val, const W *x, W *y, int xcd) {
-    if (M.nslices <= 0) return;
-    put(s, k_sub_sell<T, W>, blocks_for(M.nslices, kB / 64, 1 << 20), M, val, x, y, xcd);
-}
-template <typename T, typename W>
-void ildl_jacobi_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
-                     const T *val, const W *b, const W *xin, W *xout, int xcd) {
+void ildl_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx, const T *val,
+              const W *x, const RowOp<W> &op, int xcd) {
     if (nrows <= 0) return;
-#define JDHIP_JC(L)                                                                     \
-    put(s, k_jacobi_csr<T, W, L>, blocks_for(nrows, kB / L, 1 << 20), nrows, ptr, idx, \
-                                                                            val, b, xin, xout, xcd)
-    if (lpr >= 64) JDHIP_JC(64);
-    else if (lpr >= 32) JDHIP_JC(32);
-    else if (lpr >= 16) JDHIP_JC(16);
-    else if (lpr >= 8) JDHIP_JC(8);
-    else JDHIP_JC(4);
-#undef JDHIP_JC
-}
-template <typename T, typename W>
-void ildl_sub_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
-                  const T *val, const W *x, W *y, int xcd) {
-    if (nrows <= 0) return;
-#define JDHIP_SC(L)                                                                      \
-    put(s, k_sub_csr<T, W, L>, blocks_for(nrows, kB / L, 1 << 20), nrows, ptr, idx, val, \
-                                                                         x, y, xcd)
-    if (lpr >= 64) JDHIP_SC(64);
-    else if (lpr >= 32) JDHIP_SC(32);
-    else if (lpr >= 16) JDHIP_SC(16);
-    else if (lpr >= 8) JDHIP_SC(8);
-    else JDHIP_SC(4);
-#undef JDHIP_SC
+#define JDHIP_C(L) \
+    put(s, k_csr<T, W, L>, blocks_for(nrows, kB / L, 1 << 20), nrows, ptr, idx, val, x, op, xcd)
+    if (lpr >= 64) JDHIP_C(64);
+    else if (lpr >= 32) JDHIP_C(32);
+    else if (lpr >= 16) JDHIP_C(16);
+    else if (lpr >= 8) JDHIP_C(8);
+    else JDHIP_C(4);
+#undef JDHIP_C
 }
 template <typename T, typename W>
 void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
-                 const W *src, W *out, int xcd) {
+                 const RowOp<W> &op, int xcd) {
     if (M.nblk <= 0) return;
-    if (M.cap == 512)
-        put(s, k_stream<512, T, W>, M.nblk, M, idx, val, x, src, out, xcd);
-    else
-        put(s, k_stream<1024, T, W>, M.nblk, M, idx, val, x, src, out, xcd);
+    if (M.cap == 512) put(s, k_stream<512, T, W>, M.nblk, M, idx, val, x, op, xcd);
+    else put(s, k_stream<1024, T, W>, M.nblk, M, idx, val, x, op, xcd);
 }
 
 // Entries a block holds: 1024 where that leaves enough blocks for the 256 CUs,
@@ -526,17 +492,13 @@ void ildl_dense_gemv(const Put &s, int m, const T *Minv, const W *x, W *y) {
 #define INST(T, W)                                                                           \
     template void ildl_trsv_level<T, W>(const Put &, const int *, int, const int *,          \
                                         const int *, const T *, W *);                        \
-    template void ildl_jacobi_sweep_sell<T, W>(const Put &, const SellView &, const T *,      \
-                                               const W *, const W *, W *, int);              \
-    template void ildl_sub_sell<T, W>(const Put &, const SellView &, const T *, const W *,    \
-                                      W *, int);                                             \
-    template void ildl_jacobi_csr<T, W>(const Put &, int, int, const int *, const int *,      \
-                                        const T *, const W *, const W *, W *, int);          \
-    template void ildl_sub_csr<T, W>(const Put &, int, int, const int *, const int *,         \
-                                     const T *, const W *, W *, int);                        \
+    template void ildl_sell<T, W>(const Put &, const SellView &, const T *, const W *,        \
+                                  const RowOp<W> &, int);                                     \
+    template void ildl_csr<T, W>(const Put &, int, int, const int *, const int *, const T *,  \
+                                 const W *, const RowOp<W> &, int);                           \
     template void ildl_dense_gemv<T, W>(const Put &, int, const T *, const W *, W *);         \
-    template void ildl_stream<T, W>(const Put &, const StreamView &, const int *, const T *,   \
-                                    const W *, const W *, W *, int);
+    template void ildl_stream<T, W>(const Put &, const StreamView &, const int *, const T *,  \
+                                    const W *, const RowOp<W> &, int);
 INST(double, double)
 INST(float, double)
 INST(float, float)

@@ -59,22 +59,29 @@ struct SellView {
     const int *cbase = nullptr;
     const char *idx = nullptr;
 };
-// One Jacobi sweep of the unit triangle, xout = b - M xin.  xcd bit 0:
-// XCD-contiguous block order; bit 1: nontemporal loads of the matrix stream.
+// What a product M x becomes, row by row: v = src - (M x) (src null: 0), then
+// v = dinv v (dinv null: as it is), then v = add + v (add null: as it is),
+// rounded to the work vectors' type after each step, into out.  src, add and
+// out may be one array (a row is read and written by the same thread); out is
+// never x.  So a sweep is src = b, the last sweep before D^-1 carries dinv, the
+// last one of the second solve adds into y_B, and F x_C needs no zeroed vector.
+template <typename W>
+struct RowOp {
+    const W *src = nullptr;
+    const double *dinv = nullptr;
+    const W *add = nullptr;
+    W *out = nullptr;
+};
+// SELL-C-sigma form, one lane per row.  xcd bit 0: XCD-contiguous block order;
+// bit 1: nontemporal loads of the matrix stream.
 template <typename T, typename W>
-void ildl_jacobi_sweep_sell(const Put &s, const SellView &M, const T *val, const W *b,
-                            const W *xin, W *xout, int xcd);
-// CSR forms with lpr (4, 8, 16, 32 or 64) lanes per row, for matrices with long rows;
-// xcd != 0: XCD-contiguous block order (as for the SELL and stream forms)
+void ildl_sell(const Put &s, const SellView &M, const T *val, const W *x, const RowOp<W> &op,
+               int xcd);
+// CSR form with lpr (4, 8, 16, 32 or 64) lanes per row, for small matrices and
+// long rows; xcd != 0: XCD-contiguous block order
 template <typename T, typename W>
-void ildl_jacobi_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
-                     const T *val, const W *b, const W *xin, W *xout, int xcd);
-template <typename T, typename W>
-void ildl_sub_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx,
-                  const T *val, const W *x, W *y, int xcd);
-// y[r] -= sum_j M(r, j) x[j] over the rows of a SELL-C-sigma matrix
-template <typename T, typename W>
-void ildl_sub_sell(const Put &s, const SellView &M, const T *val, const W *x, W *y, int xcd);
+void ildl_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx, const T *val,
+              const W *x, const RowOp<W> &op, int xcd);
 // CSR-stream form: blocks of consecutive rows with at most cap - 2 entries
 // (and 256 rows) each, or one longer row, streamed through LDS with coalesced
 // loads.  The product reads the CSR's own values and columns (which end in
@@ -98,11 +105,10 @@ struct StreamHost {
     std::vector<unsigned short> off, c16;
 };
 StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx);
-// out = src - M x over every row (a sweep: src = b; a product: src = out = y).
 // xcd != 0: every XCD takes one contiguous range of row blocks.
 template <typename T, typename W>
 void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
-                 const W *src, W *out, int xcd);
+                 const RowOp<W> &op, int xcd);
 template <typename W>
 void ildl_dscale(const Put &s, int n, const double *dinv, W *x);
 // x = D^-1 x with 2x2 blocks: row i pairs with pair[i] (-1: 1x1 pivot,

@@ -61,6 +61,21 @@ def test_stream_rows_at_the_block_size(k, single):
     _check(lambda: _hub(700, k), {"ildl_form": 1}, 3, single=single)
 
 
+# one, two and three sweeps: where the last sweep carries D^-1 and the addition
+# of the second solve, with 1x1 and with 2x2 pivots, in every family of forms,
+# replayed and launched one by one
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("coupling", [0, 1])
+@pytest.mark.parametrize("form", [0, 1, 8])
+@pytest.mark.parametrize("sweeps", [1, 2, 3])
+@pytest.mark.parametrize("gen,spd", [(lambda: M.laplace((13, 11, 9)), True),
+                                     (lambda: M.anderson(11, 16.5, 4), False)])
+def test_fused_ends_of_the_sweeps(gen, spd, sweeps, form, coupling, graph):
+    for single in (False, True):
+        _check(gen, {"ildl_form": form, "ildl_graph": graph}, sweeps, coupling=coupling,
+               single=single, spd=spd, dense_max=50)
+
+
 # a level large enough for the blocks of 1022 entries
 def test_stream_wide_blocks():
     _check(lambda: M.laplace((64, 63, 61)), {"ildl_form": 1}, 2)
