@@ -42,12 +42,12 @@ struct SolverOps : Ops {
     bool mv = false, pc = false;
     bool has_matvec() const override { return mv; }
     bool has_precond() const override { return pc; }
-    void matvec(const double *x, double *y, const double *eta_dev, double eta, const double *u,
-                double *udot) override;
+    int matvec(const double *x, double *y, const double *eta_dev, double eta, const double *u,
+               double *udot) override;
     void precond(JdEngine &e, double *z, const double *r) override;
     bool f32 = false;
     bool has_f32() const override { return f32; }
-    void matvec_f(const float *x, float *y, double eta, const float *u, double *udot) override;
+    int matvec_f(const float *x, float *y, double eta, const float *u, double *udot) override;
     void precond_f(JdEngine &e, float *z, const float *r) override;
     void bmatvec(const double *x, double *y) override;
 };
@@ -221,15 +221,15 @@ struct Solver {
                   int *info, double *gap, bool internal_mv, long *ndx3 = nullptr);
 };
 
-void SolverOps::matvec(const double *x, double *y, const double *eta_dev, double eta,
-                       const double *u, double *udot) {
+int SolverOps::matvec(const double *x, double *y, const double *eta_dev, double eta,
+                      const double *u, double *udot) {
     (void)eta_dev;
-    spmv<double>(S->ctx.stream, S->ctx.rb, S->A, x, y, eta, u, udot);
+    return spmv<double>(S->ctx.stream, S->ctx.rb, S->A, x, y, eta, u, udot);
 }
 void SolverOps::precond(JdEngine &, double *z, const double *r) { S->precond_request(z, r); }
-void SolverOps::matvec_f(const float *x, float *y, double eta, const float *u, double *udot) {
+int SolverOps::matvec_f(const float *x, float *y, double eta, const float *u, double *udot) {
     S->A.f_vals64 = S->inner_spmv64;
-    spmv<float>(S->ctx.stream, S->ctx.rb, S->A, x, y, eta, u, udot);
+    return spmv<float>(S->ctx.stream, S->ctx.rb, S->A, x, y, eta, u, udot);
 }
 void SolverOps::precond_f(JdEngine &, float *z, const float *r) { S->precond_request_f(z, r); }
 void SolverOps::bmatvec(const double *x, double *y) {

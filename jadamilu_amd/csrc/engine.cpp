@@ -26,7 +26,7 @@ void DevCtx::init(int dev) {
     device = dev;
     JDHIP_CHECK(hipSetDevice(dev));
     JDHIP_CHECK(hipStreamCreate(&stream));
-    JDHIP_CHECK(hipMalloc(&rb.partials, sizeof(double) * kMaxPartials));
+    JDHIP_CHECK(hipMalloc(&rb.partials, sizeof(double) * (kMaxPartials + kInnerPartials)));
     JDHIP_CHECK(hipMalloc(&rb.counter, sizeof(unsigned) * 16));
     JDHIP_CHECK(hipMemsetAsync(rb.counter, 0, sizeof(unsigned) * 16, stream));
     JDHIP_CHECK(hipMalloc(&d_small, sizeof(double) * 8192));
@@ -77,8 +77,11 @@ void DevCtx::ensure_tmp(long len) {
 // ---------------------------------------------------------------------------
 void JdEngine::fetch(double *host, const double *dev, long cnt) {
     if (cnt <= 0) return;
-    JDHIP_CHECK(hipMemcpyAsync(ctx_->h_pin, dev, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                               ctx_->stream));
+    // by a kernel into the pinned buffer: 3 us less than a copy
+    if (cnt <= 1024) get_small(ctx_->stream, ctx_->h_pin, dev, (int)cnt);
+    else
+        JDHIP_CHECK(hipMemcpyAsync(ctx_->h_pin, dev, sizeof(double) * cnt,
+                                   hipMemcpyDeviceToHost, ctx_->stream));
     ctx_->sync();
     ++nsync;
     std::memcpy(host, ctx_->h_pin, sizeof(double) * cnt);
@@ -86,6 +89,10 @@ void JdEngine::fetch(double *host, const double *dev, long cnt) {
 
 void JdEngine::put(double *dev, const double *host, long cnt) {
     if (cnt <= 0) return;
+    if (cnt <= kMaxCols) {  // as a kernel's arguments: nothing to wait for
+        put_small(ctx_->stream, dev, host, (int)cnt);
+        return;
+    }
     std::memcpy(ctx_->h_pin + 4096, host, sizeof(double) * cnt);
     JDHIP_CHECK(hipMemcpyAsync(dev, ctx_->h_pin + 4096, sizeof(double) * cnt,
                                hipMemcpyHostToDevice, ctx_->stream));
@@ -911,9 +918,7 @@ L20:  // expansion
         h.flag = 0;
         h.ggk2 = gk * gk;
         h.eta = eta;
-        JDHIP_CHECK(hipMemcpyAsync(ctx_->d_sc, &h, sizeof(InnerScalars), hipMemcpyHostToDevice,
-                                   s));
-        ctx_->sync();
+        inner_init(s, ctx_->d_sc, h);
     }
 L10i:  // new inner iteration: preconditioner solve Z = P^-1 R
     ++ls_iter;
@@ -923,16 +928,10 @@ L10i:  // new inner iteration: preconditioner solve Z = P^-1 R
         float *xf = fbuf_ + 4L * n, *x2f = fbuf_ + 5L * n, *Qf = fbuf_ + 6L * n;
         ops_->precond_f(*this, zf, rf);
         flagcg = true;
-        cg_project_rho<float>(s, rb, zf, Qf, *neig + 1, rf, n, ctx_->d_sc, ctx_->slot(0));
-        cg_direction<float>(s, zf, pf, n, ctx_->d_sc, ls_iter);
-        ops_->matvec_f(pf, qf, eta, Qf, &ctx_->d_sc->alprho);
-        cg_project_alpha<float>(s, rb, qf, Qf, pf, n, ctx_->d_sc);
-        if (ls_posdef) {
-            cg_update_posdef<float>(s, rb, rf, qf, xf, pf, n, ctx_->d_sc);
-        } else {
-            qmr_update_r<float>(s, rb, rf, qf, n, ctx_->d_sc);
-            qmr_update_x<float>(s, rb, xf, x2f, pf, n, ctx_->d_sc, ls_iter);
-        }
+        inner_direction<float>(s, rb, zf, Qf, *neig + 1, rf, pf, n, ctx_->d_sc, ls_iter, nullptr);
+        const int np = ops_->matvec_f(pf, qf, eta, Qf, &ctx_->d_sc->alprho);
+        inner_update<float>(s, rb, ls_posdef, rf, qf, Qf, xf, x2f, pf, n, ctx_->d_sc, ls_iter, np,
+                            ctx_->h_sc);
         goto Lsync;
     }
     *ndx1 = wcg + n;  // Z
@@ -946,41 +945,29 @@ L10i:  // new inner iteration: preconditioner solve Z = P^-1 R
     return;
 L38:  // project Z against [u, X] ; rho = r.z ; direction
     flagcg = true;
-    cg_project_rho(s, rb, D(wcg + n), D(uu), *neig + 1, D(wcg), n, ctx_->d_sc, ctx_->slot(0));
-    cg_direction(s, D(wcg + n), D(wcg + 2L * n), n, ctx_->d_sc, ls_iter);
+    inner_direction(s, rb, D(wcg + n), D(uu), *neig + 1, D(wcg), D(wcg + 2L * n), n, ctx_->d_sc,
+                    ls_iter, internal_mv() ? nullptr : ctx_->h_sc);
     *ndx1 = wcg + 2L * n;  // P
     *ndx2 = wcg + 3L * n;  // Q
     rlbl = 3;
+    ls_np = 0;
     if (internal_mv()) {
-        ops_->matvec(D(*ndx1), D(*ndx2), nullptr, eta, D(bu), &ctx_->d_sc->alprho);
-        goto L37b;
+        ls_np = ops_->matvec(D(*ndx1), D(*ndx2), nullptr, eta, D(bu), &ctx_->d_sc->alprho);
+        goto L4i;
     }
     // external matvec: the breakdown test must be known before returning
-    JDHIP_CHECK(hipMemcpyAsync(ctx_->h_sc, ctx_->d_sc, sizeof(InnerScalars),
-                               hipMemcpyDeviceToHost, s));
     ctx_->sync();
     ++nsync;
     if (ctx_->h_sc->flag == 1) goto L40i;
     *ijob = 1;
     return;
 L37:  // after an external matvec: Q -= eta P ; alprho = u.Q
-    axpy(s, D(wcg + 3L * n), -eta, D(wcg + 2L * n), n);
-    multidot(s, rb, D(bu), n, 1, D(wcg + 3L * n), n, &ctx_->d_sc->alprho);
+    ls_np = inner_shift(s, rb, D(wcg + 3L * n), eta, D(wcg + 2L * n), D(bu), n);
     ++*iter;
-    goto L4i;
-L37b:
 L4i:
-    cg_project_alpha(s, rb, D(wcg + 3L * n), D(bu), D(wcg + 2L * n), n, ctx_->d_sc);
-    if (ls_posdef) {
-        cg_update_posdef(s, rb, D(wcg), D(wcg + 3L * n), D(xcg), D(wcg + 2L * n), n,
-                         ctx_->d_sc);
-    } else {
-        qmr_update_r(s, rb, D(wcg), D(wcg + 3L * n), n, ctx_->d_sc);
-        qmr_update_x(s, rb, D(xcg), D(xcg2), D(wcg + 2L * n), n, ctx_->d_sc, ls_iter);
-    }
+    inner_update(s, rb, ls_posdef, D(wcg), D(wcg + 3L * n), D(bu), D(xcg), D(xcg2),
+                 D(wcg + 2L * n), n, ctx_->d_sc, ls_iter, ls_np, ctx_->h_sc);
 Lsync:
-    JDHIP_CHECK(hipMemcpyAsync(ctx_->h_sc, ctx_->d_sc, sizeof(InnerScalars),
-                               hipMemcpyDeviceToHost, s));
     ctx_->sync();
     ++nsync;
     {

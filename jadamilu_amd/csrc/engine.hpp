@@ -72,16 +72,21 @@ class JdEngine;
 struct Ops {
     virtual ~Ops() = default;
     virtual bool has_matvec() const { return false; }
-    // y = A x ; if eta_dev/eta: y -= eta x ; if u: *udot_dev = u.y
-    virtual void matvec(const double *x, double *y, const double *eta_dev, double eta,
-                        const double *u, double *udot_dev) {}
+    // y = A x ; if eta_dev/eta: y -= eta x ; if u: u.y, in *udot_dev (0 is
+    // returned) or as that many partial sums (see spmv)
+    virtual int matvec(const double *x, double *y, const double *eta_dev, double eta,
+                       const double *u, double *udot_dev) {
+        return 0;
+    }
     virtual bool has_precond() const { return false; }
     // called when the reference would return IJOB=2 to PJDRVCOM
     virtual void precond(JdEngine &e, double *z, const double *r) {}
     // FP32 inner solver (mixed path): operator and preconditioner on float
     // vectors; only used when has_f32() and both operators are inline.
     virtual bool has_f32() const { return false; }
-    virtual void matvec_f(const float *x, float *y, double eta, const float *u, double *udot) {}
+    virtual int matvec_f(const float *x, float *y, double eta, const float *u, double *udot) {
+        return 0;
+    }
     virtual void precond_f(JdEngine &e, float *z, const float *r) {}
     // generalized problem A x = lambda B x: y = B x (inline when has_matvec)
     virtual void bmatvec(const double *x, double *y) {}
@@ -184,6 +189,7 @@ class JdEngine {
 
     // ---- LSOLREVCOM locals ----
     int ls_iter = 0, ls_maxit = 0;
+    int ls_np = 0;  // partial sums of u.q that the step's product left (see inner_update)
     bool ls_posdef = false;
 
     // ---- STOPTEST locals (SAVE) ----

@@ -16,6 +16,10 @@ constexpr int kBlock = 256;      // threads per block (4 wave64)
 constexpr int kMaxCols = 64;     // max columns of a tall-skinny product
 constexpr int kMaxRedBlocks = 4096;  // enough waves in flight to cover HBM latency
 constexpr int kMaxPartials = kMaxRedBlocks * 64;  // reduction scratch (doubles)
+// Blocks of an inner-step kernel: every block of the next kernel sums their
+// partial sums again, so there are few of them
+constexpr int kInnerBlocks = 512;
+constexpr int kInnerPartials = kInnerBlocks * (kMaxCols + 8);
 
 // Device-resident scalars of the inner solver (one per engine).
 struct InnerScalars {
@@ -30,6 +34,10 @@ struct InnerScalars {
 // Reduction scratch owned by an engine.
 struct RedBuf {
     double *partials;   // kMaxPartials
+    // the inner step's partial sums (at most kInnerBlocks of each): they follow
+    // those of the products, which begin at partials
+    double *inner(int k) const { return partials + kMaxPartials + (long)k * kInnerBlocks; }
+    double *inner_u() const { return inner(0); }
     unsigned *counter;  // 8 counters
     double *out;        // kMaxCols results
 };
@@ -101,10 +109,11 @@ struct CsrDev {
     bool f_vals64 = false;    // FP32 vectors read the double values
 };
 // y = A x (T = double: A.val, T = float: A.valf); if eta != 0: y -= eta x;
-// if u: *udot_out = u.y (double)
+// if u: u.y (double), in *udot_out, or as partial sums at rb.inner_u() where
+// there are at most kInnerBlocks of them: their number is returned, else 0
 template <typename T>
-void spmv(hipStream_t s, const RedBuf &rb, const CsrDev &A, const T *x, T *y, double eta,
-          const T *u, double *udot_out);
+int spmv(hipStream_t s, const RedBuf &rb, const CsrDev &A, const T *x, T *y, double eta,
+         const T *u, double *udot_out);
 
 // Y = A X for k vectors (column-major, leading dimensions ldx, ldy), FP64,
 // in passes of up to 8 vectors over the matrix (kernels_spmm.hip)
@@ -118,26 +127,33 @@ void convert(hipStream_t s, float *dst, const double *src, long n);
 void convert(hipStream_t s, double *dst, const float *src, long n);
 
 // ---- inner solver (LSOLREVCOM) fused steps, T = double or float ----
-// z = P^-1 r is already in z: ycoef = Q^T z ; z -= Q ycoef ; rho = r.z
+// A step is project_direction, the product Q = (A - eta) P, update; the
+// scalars stay in sc, and update leaves a copy of them in host, which is
+// pinned memory that the caller reads after it has waited for the stream.
+//
+// z = P^-1 r is already in z: z -= Q Q^T z (jq columns); rho = r.z, breakdown
+// test (flag 1); z += (rho/rho1) p; p = z.  iter: the iteration number.  host
+// (may be null): sc's flag is left there too.
 template <typename T>
-void cg_project_rho(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, const T *r,
-                    long n, InnerScalars *sc, double *ycoef);
-// z += (rho/rho1) p ; p = z   (iteration number from the host)
+void inner_direction(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, const T *r, T *p,
+                     long n, InnerScalars *sc, int iter, InnerScalars *host);
+// q = (A - eta) p; np = 0: sc->alprho = u.q is known, np > 0: as np partial
+// sums at rb.inner_u().  Then q -= u alprho, pq = p.q, alpha (breakdown: flag
+// 2), and PCG's r -= alpha q, x += alpha p, |r|^2, |x|^2, or (posdef = false)
+// sQMR's smoothed update of x and x2.
 template <typename T>
-void cg_direction(hipStream_t s, T *z, T *p, long n, InnerScalars *sc, int iter);
-// q already = (A - eta) p, alprho = u.q ; q -= u alprho ; pq = p.q ; alpha
-template <typename T>
-void cg_project_alpha(hipStream_t s, const RedBuf &rb, T *q, const T *u, const T *p, long n,
-                      InnerScalars *sc);
-// PCG: r -= alpha q ; gk2 = r.r ; x += alpha p ; xn2 = x.x
-template <typename T>
-void cg_update_posdef(hipStream_t s, const RedBuf &rb, T *r, const T *q, T *x, const T *p,
-                      long n, InnerScalars *sc);
-// sQMR: r -= alpha q ; gk2 ; smoothing scalars ; then x, x2 update
-template <typename T>
-void qmr_update_r(hipStream_t s, const RedBuf &rb, T *r, const T *q, long n, InnerScalars *sc);
-template <typename T>
-void qmr_update_x(hipStream_t s, const RedBuf &rb, T *x, T *x2, const T *p, long n,
-                  InnerScalars *sc, int iter);
+void inner_update(hipStream_t s, const RedBuf &rb, bool posdef, T *r, T *q, const T *u, T *x,
+                  T *x2, const T *p, long n, InnerScalars *sc, int iter, int np,
+                  InnerScalars *host);
+// q -= eta p and the partial sums of u.q at rb.inner_u(), after a product that
+// the caller made; returns their number
+int inner_shift(hipStream_t s, const RedBuf &rb, double *q, double eta, const double *p,
+                const double *u, long n);
+// sc = *h (by value: no copy, no wait)
+void inner_init(hipStream_t s, InnerScalars *sc, const InnerScalars &h);
+// dst[0..cnt) = src[0..cnt) by a kernel: into pinned memory, or (put_small, cnt
+// <= kMaxCols) from the host's values by value
+void get_small(hipStream_t s, double *host, const double *dev, int cnt);
+void put_small(hipStream_t s, double *dev, const double *host, int cnt);
 
 }  // namespace jdhip

@@ -61,11 +61,20 @@ __global__ __launch_bounds__(kBlock) void k_gemv_n(double *__restrict__ w,
     if ((int)threadIdx.x < jv) ys[threadIdx.x] = alpha * y[threadIdx.x];
     __syncthreads();
     double acc[1] = {0.0};
+    // eight columns' loads at a time, without a branch between them
+    constexpr int CH = NC < 8 ? NC : 8;
     for (long i = blockIdx.x * (long)kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock) {
         double wi = (beta == 0.0) ? 0.0 : (beta == 1.0 ? w[i] : beta * w[i]);
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-            if (c < jv) wi += ys[c] * V[c * ldv + i];
+        for (int c0 = 0; c0 < NC; c0 += CH) {
+            if (c0 >= jv) break;
+            double v[CH];
+#pragma unroll
+            for (int c = 0; c < CH; ++c) v[c] = V[(long)min(c0 + c, jv - 1) * ldv + i];
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+                if (c0 + c < jv) wi += ys[c0 + c] * v[c];
+        }
         w[i] = wi;
         if (NORM) acc[0] += wi * wi;
     }
