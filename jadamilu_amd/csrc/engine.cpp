@@ -38,6 +38,8 @@ void DevCtx::init(int dev) {
     JDHIP_CHECK(hipHostMalloc(&h_pin, sizeof(double) * 8192, hipHostMallocDefault));
     JDHIP_CHECK(hipHostMalloc(&h_sc, sizeof(InnerScalars), hipHostMallocDefault));
     std::memset(h_sc, 0, sizeof(InnerScalars));
+    JDHIP_CHECK(hipHostMalloc(&h_seq, sizeof(unsigned), hipHostMallocDefault));
+    *h_seq = 0;
     JDHIP_CHECK(hipMalloc(&d_gram, sizeof(double) * kGramScratch));
     JDHIP_CHECK(hipMalloc(&d_gout, sizeof(double) * kMaxCols * kMaxCols));
     JDHIP_CHECK(hipEventCreateWithFlags(&ev_sync, hipEventBlockingSync | hipEventDisableTiming));
@@ -56,6 +58,7 @@ void DevCtx::release() {
     hipFree(d_gout);
     hipHostFree(h_pin);
     hipHostFree(h_sc);
+    hipHostFree(h_seq);
     if (ev_sync) hipEventDestroy(ev_sync);
     ev_sync = nullptr;
     hipStreamDestroy(stream);
@@ -78,11 +81,15 @@ void DevCtx::ensure_tmp(long len) {
 void JdEngine::fetch(double *host, const double *dev, long cnt) {
     if (cnt <= 0) return;
     // by a kernel into the pinned buffer: 3 us less than a copy
-    if (cnt <= 1024) get_small(ctx_->stream, ctx_->h_pin, dev, (int)cnt);
-    else
+    if (cnt <= 1024) {
+        const Done d = ctx_->next_done();
+        get_small(ctx_->stream, ctx_->h_pin, dev, (int)cnt, d);
+        ctx_->wait(d);
+    } else {
         JDHIP_CHECK(hipMemcpyAsync(ctx_->h_pin, dev, sizeof(double) * cnt,
                                    hipMemcpyDeviceToHost, ctx_->stream));
-    ctx_->sync();
+        ctx_->sync();
+    }
     ++nsync;
     std::memcpy(host, ctx_->h_pin, sizeof(double) * cnt);
 }
@@ -928,10 +935,10 @@ L10i:  // new inner iteration: preconditioner solve Z = P^-1 R
         float *xf = fbuf_ + 4L * n, *x2f = fbuf_ + 5L * n, *Qf = fbuf_ + 6L * n;
         ops_->precond_f(*this, zf, rf);
         flagcg = true;
-        inner_direction<float>(s, rb, zf, Qf, *neig + 1, rf, pf, n, ctx_->d_sc, ls_iter, nullptr);
+        inner_direction<float>(s, rb, zf, Qf, *neig + 1, rf, pf, n, ctx_->d_sc, ls_iter);
         const int np = ops_->matvec_f(pf, qf, eta, Qf, &ctx_->d_sc->alprho);
         inner_update<float>(s, rb, ls_posdef, rf, qf, Qf, xf, x2f, pf, n, ctx_->d_sc, ls_iter, np,
-                            ctx_->h_sc);
+                            ctx_->h_sc, step_done = ctx_->next_done());
         goto Lsync;
     }
     *ndx1 = wcg + n;  // Z
@@ -946,7 +953,7 @@ L10i:  // new inner iteration: preconditioner solve Z = P^-1 R
 L38:  // project Z against [u, X] ; rho = r.z ; direction
     flagcg = true;
     inner_direction(s, rb, D(wcg + n), D(uu), *neig + 1, D(wcg), D(wcg + 2L * n), n, ctx_->d_sc,
-                    ls_iter, internal_mv() ? nullptr : ctx_->h_sc);
+                    ls_iter);
     *ndx1 = wcg + 2L * n;  // P
     *ndx2 = wcg + 3L * n;  // Q
     rlbl = 3;
@@ -955,8 +962,11 @@ L38:  // project Z against [u, X] ; rho = r.z ; direction
         ls_np = ops_->matvec(D(*ndx1), D(*ndx2), nullptr, eta, D(bu), &ctx_->d_sc->alprho);
         goto L4i;
     }
-    // external matvec: the breakdown test must be known before returning
-    ctx_->sync();
+    // external matvec: the breakdown test must be known before returning, and
+    // P be written (for a caller on another stream, too)
+    step_done = ctx_->next_done();
+    inner_flag(s, ctx_->d_sc, ctx_->h_sc, step_done);
+    ctx_->wait(step_done);
     ++nsync;
     if (ctx_->h_sc->flag == 1) goto L40i;
     *ijob = 1;
@@ -966,9 +976,10 @@ L37:  // after an external matvec: Q -= eta P ; alprho = u.Q
     ++*iter;
 L4i:
     inner_update(s, rb, ls_posdef, D(wcg), D(wcg + 3L * n), D(bu), D(xcg), D(xcg2),
-                 D(wcg + 2L * n), n, ctx_->d_sc, ls_iter, ls_np, ctx_->h_sc);
+                 D(wcg + 2L * n), n, ctx_->d_sc, ls_iter, ls_np, ctx_->h_sc,
+                 step_done = ctx_->next_done());
 Lsync:
-    ctx_->sync();
+    ctx_->wait(step_done);
     ++nsync;
     {
         const InnerScalars &h = *ctx_->h_sc;

@@ -61,6 +61,28 @@ struct DevCtx {
             JDHIP_CHECK(hipStreamSynchronize(stream));
         }
     }
+    // Wait for the last kernel on the stream, which stores the number of
+    // next_done() behind what it leaves in pinned memory: every kernel before
+    // it has then ended.  Polling that number takes 27 us for eight launches
+    // and the wait, hipStreamSynchronize 53 us.  A wait of more than 20 ms (a
+    // long apply, or an error, which only the runtime reports) goes on there.
+    unsigned *h_seq = nullptr;
+    unsigned seq = 0;
+    Done next_done() { return {h_seq, ++seq}; }
+    void wait(Done d) {
+        if (!blocking_sync) {
+            const auto t0 = std::chrono::steady_clock::now();
+            for (unsigned spin = 0;; ++spin) {
+                if (__atomic_load_n(d.seq, __ATOMIC_ACQUIRE) == d.v) return;
+                if ((spin & 255) == 255 &&
+                    std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20))
+                    break;
+            }
+        }
+        sync();
+        if (__atomic_load_n(d.seq, __ATOMIC_ACQUIRE) != d.v)
+            throw std::runtime_error("HIP error: a kernel of the step did not run");
+    }
     // device slots
     double *slot(int k) { return d_small + (long)k * kMaxCols; }
 };
@@ -189,6 +211,7 @@ class JdEngine {
 
     // ---- LSOLREVCOM locals ----
     int ls_iter = 0, ls_maxit = 0;
+    Done step_done{};  // the end of the inner step in flight
     int ls_np = 0;  // partial sums of u.q that the step's product left (see inner_update)
     bool ls_posdef = false;
 

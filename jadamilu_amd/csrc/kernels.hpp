@@ -126,17 +126,25 @@ void diag_apply(hipStream_t s, T *z, const T *d, const T *r, long n);
 void convert(hipStream_t s, float *dst, const double *src, long n);
 void convert(hipStream_t s, double *dst, const float *src, long n);
 
+// Where a kernel tells the host that it has finished writing to pinned memory:
+// it stores v at seq (see DevCtx::wait).
+struct Done {
+    unsigned *seq;
+    unsigned v;
+};
+
 // ---- inner solver (LSOLREVCOM) fused steps, T = double or float ----
 // A step is project_direction, the product Q = (A - eta) P, update; the
 // scalars stay in sc, and update leaves a copy of them in host, which is
 // pinned memory that the caller reads after it has waited for the stream.
 //
 // z = P^-1 r is already in z: z -= Q Q^T z (jq columns); rho = r.z, breakdown
-// test (flag 1); z += (rho/rho1) p; p = z.  iter: the iteration number.  host
-// (may be null): sc's flag is left there too.
+// test (flag 1); z += (rho/rho1) p; p = z.  iter: the iteration number.
 template <typename T>
 void inner_direction(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, const T *r, T *p,
-                     long n, InnerScalars *sc, int iter, InnerScalars *host);
+                     long n, InnerScalars *sc, int iter);
+// sc's flag into host, behind everything on the stream
+void inner_flag(hipStream_t s, const InnerScalars *sc, InnerScalars *host, Done done);
 // q = (A - eta) p; np = 0: sc->alprho = u.q is known, np > 0: as np partial
 // sums at rb.inner_u().  Then q -= u alprho, pq = p.q, alpha (breakdown: flag
 // 2), and PCG's r -= alpha q, x += alpha p, |r|^2, |x|^2, or (posdef = false)
@@ -144,7 +152,7 @@ void inner_direction(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, 
 template <typename T>
 void inner_update(hipStream_t s, const RedBuf &rb, bool posdef, T *r, T *q, const T *u, T *x,
                   T *x2, const T *p, long n, InnerScalars *sc, int iter, int np,
-                  InnerScalars *host);
+                  InnerScalars *host, Done done);
 // q -= eta p and the partial sums of u.q at rb.inner_u(), after a product that
 // the caller made; returns their number
 int inner_shift(hipStream_t s, const RedBuf &rb, double *q, double eta, const double *p,
@@ -153,7 +161,7 @@ int inner_shift(hipStream_t s, const RedBuf &rb, double *q, double eta, const do
 void inner_init(hipStream_t s, InnerScalars *sc, const InnerScalars &h);
 // dst[0..cnt) = src[0..cnt) by a kernel: into pinned memory, or (put_small, cnt
 // <= kMaxCols) from the host's values by value
-void get_small(hipStream_t s, double *host, const double *dev, int cnt);
+void get_small(hipStream_t s, double *host, const double *dev, int cnt, Done done);
 void put_small(hipStream_t s, double *dev, const double *host, int cnt);
 
 }  // namespace jdhip

@@ -349,14 +349,12 @@ __global__ __launch_bounds__(kBlock) void k_project_rho(T *__restrict__ z,
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_direction(T *__restrict__ z, T *__restrict__ p,
                                                       long n, InnerScalars *sc, int iter,
-                                                      const double *__restrict__ prho,
-                                                      InnerScalars *host) {
+                                                      const double *__restrict__ prho) {
     const double rho = block_total(prho, gridDim.x);
     const bool bad = broke(sc, rho);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc->rho = rho;
         sc->flag = bad ? 1 : 0;
-        if (host) host->flag = bad ? 1 : 0;
     }
     if (bad) return;
     const bool first = iter <= 1;
@@ -491,7 +489,7 @@ __global__ __launch_bounds__(kBlock) void k_qmr_x(T *__restrict__ x, T *__restri
 // ||r||^2, then those of ||x||^2.
 __global__ __launch_bounds__(kBlock) void k_inner_end(InnerScalars *sc, bool posdef,
                                                       const double *__restrict__ pout, int np,
-                                                      InnerScalars *host) {
+                                                      InnerScalars *host, Done done) {
     const bool on = !sc->flag;
     const bool bad = on && broke(sc, sc->pq);
     double rr = 0.0, xx = 0.0;
@@ -517,13 +515,14 @@ __global__ __launch_bounds__(kBlock) void k_inner_end(InnerScalars *sc, bool pos
     }
     *sc = h;
     *host = h;
+    __hip_atomic_store(done.seq, done.v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 static inline int inner_grid(long n) { return grid_for(n, kBlock, kInnerBlocks); }
 
 template <typename T>
 void inner_direction(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, const T *r, T *p,
-                     long n, InnerScalars *sc, int iter, InnerScalars *host) {
+                     long n, InnerScalars *sc, int iter) {
     const int g = inner_grid(n);
     double *py = rb.inner(8), *prho = rb.inner(1);
 #define JDHIP_PR(NC)                                                                    \
@@ -539,13 +538,21 @@ void inner_direction(hipStream_t s, const RedBuf &rb, T *z, const T *Q, int jq, 
     else if (jq <= 32) JDHIP_PR(32);
     else JDHIP_PR(64);
 #undef JDHIP_PR
-    k_direction<T><<<g, kBlock, 0, s>>>(z, p, n, sc, iter, prho, host);
+    k_direction<T><<<g, kBlock, 0, s>>>(z, p, n, sc, iter, prho);
+}
+
+__global__ void k_inner_flag(const InnerScalars *sc, InnerScalars *host, Done done) {
+    host->flag = sc->flag;
+    __hip_atomic_store(done.seq, done.v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+void inner_flag(hipStream_t s, const InnerScalars *sc, InnerScalars *host, Done done) {
+    k_inner_flag<<<1, 1, 0, s>>>(sc, host, done);
 }
 
 template <typename T>
 void inner_update(hipStream_t s, const RedBuf &rb, bool posdef, T *r, T *q, const T *u, T *x,
                   T *x2, const T *p, long n, InnerScalars *sc, int iter, int np,
-                  InnerScalars *host) {
+                  InnerScalars *host, Done done) {
     const int g = inner_grid(n);
     double *ppq = rb.inner(1), *pout = rb.inner(2);
     k_project_alpha<T><<<g, kBlock, 0, s>>>(q, u, p, n, sc, rb.inner_u(), np, ppq);
@@ -555,7 +562,7 @@ void inner_update(hipStream_t s, const RedBuf &rb, bool posdef, T *r, T *q, cons
         k_qmr_r<T><<<g, kBlock, 0, s>>>(r, q, n, sc, ppq, pout);
         k_qmr_x<T><<<g, kBlock, 0, s>>>(x, x2, p, n, sc, iter, pout, pout + g);
     }
-    k_inner_end<<<1, kBlock, 0, s>>>(sc, posdef, pout, g, host);
+    k_inner_end<<<1, kBlock, 0, s>>>(sc, posdef, pout, g, host, done);
 }
 
 __global__ __launch_bounds__(kBlock) void k_inner_shift(double *__restrict__ q, double eta,
@@ -595,11 +602,15 @@ void put_small(hipStream_t s, double *dev, const double *host, int cnt) {
     k_put<<<1, kMaxCols, 0, s>>>(dev, h, cnt);
 }
 __global__ __launch_bounds__(kBlock) void k_get(double *host, const double *__restrict__ dev,
-                                                int cnt) {
+                                                int cnt, Done done) {
     for (int i = threadIdx.x; i < cnt; i += kBlock) host[i] = dev[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(done.seq, done.v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-void get_small(hipStream_t s, double *host, const double *dev, int cnt) {
-    k_get<<<1, kBlock, 0, s>>>(host, dev, cnt);
+void get_small(hipStream_t s, double *host, const double *dev, int cnt, Done done) {
+    k_get<<<1, kBlock, 0, s>>>(host, dev, cnt, done);
 }
 
 #define JDHIP_INST(T)                                                                          \
@@ -609,11 +620,10 @@ void get_small(hipStream_t s, double *host, const double *dev, int cnt) {
                          const T *, double *);                                                 \
     template void diag_apply<T>(hipStream_t, T *, const T *, const T *, long);                 \
     template void inner_direction<T>(hipStream_t, const RedBuf &, T *, const T *, int,         \
-                                     const T *, T *, long, InnerScalars *, int,                \
-                                     InnerScalars *);                                          \
+                                     const T *, T *, long, InnerScalars *, int);                                          \
     template void inner_update<T>(hipStream_t, const RedBuf &, bool, T *, T *, const T *, T *, \
                                   T *, const T *, long, InnerScalars *, int, int,              \
-                                  InnerScalars *);
+                                  InnerScalars *, Done);
 JDHIP_INST(double)
 JDHIP_INST(float)
 
