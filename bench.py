@@ -676,8 +676,9 @@ def main():
     roof_spmv = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                  "frac": achieved / HBM_PEAK_GBS, "traffic": traffic.get("spmv"),
                  "traffic_source": tsrc if traffic.get("spmv") else None,
-                 "kernel": "k_spmv_sell (symmetric SpMV, sliced ELL)" if r.stats.get(
-                     "spmv_lanes") == 0 else "k_spmv (symmetric SpMV, CSR)",
+                 "kernel": {-2: "k_spmv_dia (symmetric SpMV, upper diagonals)",
+                            0: "k_spmv_sell (symmetric SpMV, sliced ELL)"}.get(
+                     r.stats.get("spmv_lanes"), "k_spmv (symmetric SpMV, CSR)"),
                  "alg_bytes": alg, "avg_ms": spmv_ms}
     roofline = roof_spmv
     if args.precond == "ildl" and k_sw > 0:

@@ -295,8 +295,9 @@ int jdhip_pjd_batch_opts(int device, int nitems, jdhip_batch_item *items, int nw
 
 /* ---- symmetric SpMV (MATVECA, JDaux.F:3397-3418) ------------------------- */
 /* Upload a 1-based upper-triangle CSR (diagonal anywhere in each row) as the
- * device operator of ctx; 0 on success.  lanes_per_row: 0 = autotune (the
- * formats below timed on this matrix), -1 = sliced ELL (64-row slices, one
+ * device operator of ctx; 0 on success.  lanes_per_row: 0 = chosen (for
+ * at least 4,096 rows on at most 16 upper diagonals, one array per diagonal of
+ * the upper triangle; else the formats below timed on this matrix), -1 = sliced ELL (64-row slices, one
  * lane per row, 16-bit column offsets where a slice allows), k > 0 = CSR with
  * k lanes per row. */
 int jdhip_set_matrix(jdhip_ctx *ctx, int n, const int *ia, const int *ja, const double *a,
@@ -476,7 +477,7 @@ typedef struct {
     long inner_iters;     /* inner PCG/sQMR steps of the last call */
     long host_syncs;      /* host<->device synchronisations of the last call */
     int n_precond_setups; /* preconditioner (re)factorisations */
-    int spmv_lanes;       /* SpMV format chosen: k lanes per row, 0 sliced ELL */
+    int spmv_lanes;       /* SpMV format chosen: k lanes per row, 0 sliced ELL, -2 diagonals */
     double setup_shifts[64];
     double precond_seconds; /* host factorisation + upload time of the last call */
     double fill;            /* stored factor entries / nnz(upper A) (ILDL) */

@@ -142,7 +142,8 @@ struct Solver {
         if (M.val) hipFree(M.val);
         if (M.valf) hipFree(M.valf);
         for (void *p : {(void *)M.s_vptr, (void *)M.s_iptr, (void *)M.s_wm, (void *)M.s_val,
-                        (void *)M.s_valf, (void *)M.s_idx})
+                        (void *)M.s_valf, (void *)M.s_idx, (void *)M.dia.val,
+                        (void *)M.dia.valf, (void *)M.dia.mask})
             if (p) hipFree(p);
         M = CsrDev{};
     }
@@ -177,6 +178,7 @@ struct Solver {
     }
     void upload_csr(CsrDev &M, int n_, const int *ia_, const int *ja_, const double *a_,
                     int lpr);
+    bool build_dia(CsrDev &M, int n_, const int *ia_, const int *ja_, const double *a_);
     void build_sell(CsrDev &M, int n_, const std::vector<int> &rp, const std::vector<int> &col,
                     const std::vector<double> &val);
     double A_fp = 0.0;
@@ -291,10 +293,34 @@ void Solver::upload_csr(CsrDev &A, int n_, const int *ia_, const int *ja_, const
     }
     A.n = n_;
     A.nnz = nnz;
+    // Few diagonals: that form, without timing (kernels_dia.hip has both
+    // sides), and no sliced-ELL copy.  Below 4,096 rows a product is its launch
+    // in any format, and autotune_lpr keeps the CSR one.
+    if (lpr == 0 && n_ >= 4096 && build_dia(A, n_, ia_, ja_, a_)) {
+        A.lpr = kLprDia;
+        return;
+    }
     build_sell(A, n_, cnt, col, val);
     A.lpr = lpr > 0 ? lpr : 8;
     if (lpr < 0 && A.nslices > 0) A.lpr = 0;
     if (lpr == 0) A.lpr = autotune_lpr(A);
+}
+
+bool Solver::build_dia(CsrDev &A, int n_, const int *ia_, const int *ja_, const double *a_) {
+    DiaHost h;
+    if (!jdhip::build_dia(n_, ia_, ja_, a_, h)) return false;
+    JDHIP_CHECK(hipMalloc(&A.dia.val, sizeof(double) * h.val.size()));
+    JDHIP_CHECK(hipMalloc(&A.dia.valf, sizeof(float) * h.val.size()));
+    JDHIP_CHECK(hipMalloc(&A.dia.mask, sizeof(unsigned long long) * h.mask.size()));
+    h2d(ctx.stream, A.dia.val, h.val.data(), sizeof(double) * h.val.size());
+    h2d(ctx.stream, A.dia.mask, h.mask.data(), sizeof(unsigned long long) * h.mask.size());
+    convert(ctx.stream, A.dia.valf, A.dia.val, (long)h.val.size());
+    A.dia.nd = h.nd;
+    A.dia.n = n_;
+    A.dia.nslices = h.nslices;
+    A.dia.stride = h.stride;
+    std::copy(h.off.begin(), h.off.end(), A.dia.off);
+    return true;
 }
 
 // Sliced-ELL copy of the full CSR: slices of 64 rows, entries of slice s at
@@ -1245,7 +1271,10 @@ int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value) {
         S.ildl_coupling = (int)value;
     }
     else if (k == "ildl_dense_max") S.ildl_dense_max = (int)value;
-    else if (k == "spmv_lanes") S.A.lpr = (int)value;
+    else if (k == "spmv_lanes") {
+        S.A.lpr = (int)value;
+        if (S.A.lpr == 0 && S.A.nslices == 0 && S.A.dia.nd > 0) S.A.lpr = jdhip::kLprDia;
+    }
     else if (k == "inner_fp32") S.inner_fp32 = value != 0.0;
     else if (k == "inner_spmv64") S.inner_spmv64 = value != 0.0;
     else if (k == "ildl_storage") S.ildl_storage = (int)value;

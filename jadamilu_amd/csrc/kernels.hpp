@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cstdint>
+#include <vector>
 
 namespace jdhip {
 
@@ -85,6 +86,40 @@ int tall_gemm_mfma(hipStream_t s, const double *V, long ldv, int K, const double
 void argmax_abs(hipStream_t s, const RedBuf &rb, const double *x, long n, double *out);
 
 // ---- sparse ----
+// Diagonal form (kernels_dia.hip): the upper triangle as one array per
+// diagonal, val[k*stride + i] = A(i, i + off[k]), off ascending from 0; for
+// slice s of 64 rows and diagonal k, mask[2*(s*nd + k)] has the rows with an
+// entry A(i, i + off[k]) and the next word those with A(i, i - off[k]).
+constexpr int kDiaMax = 16;  // most diagonals of the upper triangle
+// most rows: byte offsets of 32 bits, and a partial sum of u.y per 256 rows
+constexpr int kDiaRows = kMaxPartials * 256;
+struct DiaDev {
+    int nd = 0, n = 0, nslices = 0;
+    long stride = 0;
+    double *val = nullptr;
+    float *valf = nullptr;  // FP32 copy
+    unsigned long long *mask = nullptr;
+    long off[kDiaMax] = {};
+};
+struct DiaHost {
+    int nd = 0, nslices = 0;
+    long stride = 0;
+    std::vector<long> off;
+    std::vector<double> val;
+    std::vector<unsigned long long> mask;
+};
+// false: the matrix does not have that form
+bool build_dia(int n, const int *ia, const int *ja, const double *a, DiaHost &h);
+// (vals64: FP32 vectors with the FP64 values)
+template <typename T>
+int spmv_dia(hipStream_t s, const RedBuf &rb, const DiaDev &A, bool vals64, const T *x, T *y,
+             double eta, const T *u, double *udot_out);
+void spmm_dia(hipStream_t s, const DiaDev &A, int k, const double *x, long ldx, double *y,
+              long ldy);
+// out[0] = the sum of np partial sums
+void finish_sum(hipStream_t s, const double *partials, int np, double *out);
+
+constexpr int kLprDia = -2;
 struct CsrDev {
     int n = 0;
     long nnz = 0;
@@ -92,7 +127,8 @@ struct CsrDev {
     int *col = nullptr;
     double *val = nullptr;
     float *valf = nullptr;  // optional FP32 copy
-    int lpr = 8;            // lanes per row (CSR kernel); 0: sliced-ELL kernel
+    int lpr = 8;            // lanes per row (CSR kernel); 0: sliced-ELL kernel, kLprDia: dia
+    DiaDev dia;             // nd = 0: none
     // Sliced ELL (slices of 64 consecutive rows, one wave64 per slice, one
     // lane per row, entries of a slice stored column-major so every load of
     // the wave is contiguous).  Column indices are 16-bit offsets from the

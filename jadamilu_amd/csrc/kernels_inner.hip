@@ -59,6 +59,10 @@ __global__ __launch_bounds__(kBlock) void k_finish_columns(const double *__restr
     }
 }
 
+void finish_sum(hipStream_t s, const double *partials, int np, double *out) {
+    k_finish_columns<<<1, kBlock, 0, s>>>(partials, np, out);
+}
+
 template <typename T>
 void multidot(hipStream_t s, const RedBuf &rb, const T *V, long ldv, int jv, const T *w, long n,
               double *out) {
@@ -228,6 +232,8 @@ static int spmv_vals(hipStream_t s, const RedBuf &rb, const CsrDev &A, const TA 
 template <typename T>
 int spmv(hipStream_t s, const RedBuf &rb, const CsrDev &A, const T *x, T *y, double eta,
          const T *u, double *udot_out) {
+    if (A.lpr == kLprDia && A.dia.nd > 0)
+        return spmv_dia<T>(s, rb, A.dia, A.f_vals64, x, y, eta, u, udot_out);
     if constexpr (sizeof(T) == 8)
         return spmv_vals<T, double>(s, rb, A, A.val, A.s_val, x, y, eta, u, udot_out);
     else if (A.f_vals64)

@@ -106,6 +106,10 @@ void spmm_pass(hipStream_t s, const CsrDev &A, const double *x, long ldx, double
 
 void spmm(hipStream_t s, const CsrDev &A, int k, const double *x, long ldx, double *y,
           long ldy) {
+    if (A.lpr == kLprDia && A.dia.nd > 0) {
+        spmm_dia(s, A.dia, k, x, ldx, y, ldy);
+        return;
+    }
     for (int j0 = 0; j0 < k; j0 += 8) {
         const int kb = std::min(8, k - j0);
         const double *xj = x + (long)j0 * ldx;
