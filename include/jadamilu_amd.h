@@ -448,7 +448,7 @@ int jdhip_ildl_level_sweeps(jdhip_ctx *ctx, int *out, int cap);
 /* Kernel form of each product of each sparse level, four per level (forward
  * sweep over L_B, backward sweep over L_B^T, L_CB product, L_CB^T product):
  * 0 one lane per row on a SELL-C-sigma copy, 1 CSR-stream (row blocks of at
- * most 1022 entries staged through LDS), k >= 4 CSR with k lanes per row.
+ * most 1024 entries staged through LDS), k >= 4 CSR with k lanes per row.
  * Chosen by timing at set-up (option ildl_autotune, default 1), else by the
  * average row length.  Fills out[0..cap-1]; returns the number of levels, or
  * -1 without an ILDL preconditioner.  No reference counterpart. */

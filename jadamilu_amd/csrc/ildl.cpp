@@ -25,13 +25,11 @@ namespace {
 // Copies run on the context's stream and are waited for (the source is a
 // temporary): the legacy null stream would wait for every other context's
 // stream in the process and break another thread's graph capture.
-// pad: spare entries behind the array, zero.
 template <typename X>
-X *dev_upload(hipStream_t s, const std::vector<X> &h, size_t pad = 0) {
+X *dev_upload(hipStream_t s, const std::vector<X> &h) {
     X *p = nullptr;
-    size_t bytes = sizeof(X) * std::max<size_t>(h.size() + pad, 1);
+    size_t bytes = sizeof(X) * std::max<size_t>(h.size(), 1);
     JDHIP_CHECK(hipMalloc(&p, bytes));
-    if (pad) JDHIP_CHECK(hipMemsetAsync(p + h.size(), 0, sizeof(X) * pad, s));
     if (!h.empty()) {
         JDHIP_CHECK(hipMemcpyAsync(p, h.data(), sizeof(X) * h.size(), hipMemcpyHostToDevice, s));
         JDHIP_CHECK(hipStreamSynchronize(s));
@@ -239,7 +237,7 @@ struct DevLevel {
     int *lct_ptr = nullptr, *lct_idx = nullptr;
     T *lct_val = nullptr;
     // row blocks of the CSR-stream form for L_B, L_B^T, L_CB, L_CB^T
-    StreamView st_b, st_t, st_c, st_ct;
+    StreamView<T> st_b, st_t, st_c, st_ct;
     std::vector<int> fwd_ptr, bwd_ptr;  // host level pointers
     int *fwd_rows = nullptr, *bwd_rows = nullptr;
     W *buf = nullptr, *out = nullptr, *t1 = nullptr, *t2 = nullptr;  // work vectors
@@ -360,16 +358,16 @@ class IldlImpl : public IldlImplBase {
             sort_rows(nB, bp, bi, bv);
             sort_rows(nC, cp, ci, cv);
             D.lb_ptr = track(dev_upload(ctx_->stream, bp));
-            D.lb_idx = track(dev_upload(ctx_->stream, bi, kStreamPad));
-            D.lb_val = track(dev_upload(ctx_->stream, bv, kStreamPad));
+            D.lb_idx = track(dev_upload(ctx_->stream, bi));
+            D.lb_val = track(dev_upload(ctx_->stream, bv));
             std::vector<int> tp, ti;
             std::vector<T> tv;
             transpose(nB, nB, bp, bi, bv, tp, ti, tv);
             D.lt_ptr = track(dev_upload(ctx_->stream, tp));
-            D.lt_idx = track(dev_upload(ctx_->stream, ti, kStreamPad));
-            D.lt_val = track(dev_upload(ctx_->stream, tv, kStreamPad));
-            D.st_b = upload_stream(nB, bp, bi);
-            D.st_t = upload_stream(nB, tp, ti);
+            D.lt_idx = track(dev_upload(ctx_->stream, ti));
+            D.lt_val = track(dev_upload(ctx_->stream, tv));
+            D.st_b = upload_stream(nB, bp, bi, bv);
+            D.st_t = upload_stream(nB, tp, ti, tv);
             D.sf = upload_sell(build_sell(nB, bp, bi, bv, sigma_));
             D.sb = upload_sell(build_sell(nB, tp, ti, tv, sigma_));
             // dependency levels from the triangular (factor) numbering
@@ -386,17 +384,17 @@ class IldlImpl : public IldlImplBase {
             }
             D.sc = upload_sell(build_sell(nC, cp, ci, cv, sigma_, true));
             D.lc_ptr = track(dev_upload(ctx_->stream, cp));
-            D.lc_idx = track(dev_upload(ctx_->stream, ci, kStreamPad));
-            D.lc_val = track(dev_upload(ctx_->stream, cv, kStreamPad));
-            D.st_c = upload_stream(nC, cp, ci);
+            D.lc_idx = track(dev_upload(ctx_->stream, ci));
+            D.lc_val = track(dev_upload(ctx_->stream, cv));
+            D.st_c = upload_stream(nC, cp, ci, cv);
             D.wc = pick_form((long)ci.size(), nC);
             D.wf = D.wb = pick_form((long)bi.size(), nB);
             transpose(nC, nB, cp, ci, cv, tp, ti, tv);
             D.sct = upload_sell(build_sell(nB, tp, ti, tv, sigma_, true));
             D.lct_ptr = track(dev_upload(ctx_->stream, tp));
-            D.lct_idx = track(dev_upload(ctx_->stream, ti, kStreamPad));
-            D.lct_val = track(dev_upload(ctx_->stream, tv, kStreamPad));
-            D.st_ct = upload_stream(nB, tp, ti);
+            D.lct_idx = track(dev_upload(ctx_->stream, ti));
+            D.lct_val = track(dev_upload(ctx_->stream, tv));
+            D.st_ct = upload_stream(nB, tp, ti, tv);
             D.wct = pick_form((long)ti.size(), nB);
             D.buf = track(dev_alloc<W>(n));
             D.out = track(dev_alloc<W>(n));
@@ -600,16 +598,18 @@ class IldlImpl : public IldlImplBase {
         return v;
     }
 
-    StreamView upload_stream(int nrows, const std::vector<int> &ptr,
-                             const std::vector<int> &idx) {
-        const StreamHost h = build_stream(nrows, ptr, idx);
-        StreamView v;
+    StreamView<T> upload_stream(int nrows, const std::vector<int> &ptr,
+                                const std::vector<int> &idx, const std::vector<T> &val) {
+        const StreamHost<T> h = build_stream(nrows, ptr, idx, val);
+        StreamView<T> v;
         v.nblk = (int)h.desc.size();
         v.cap = h.cap;
         v.desc = track(dev_upload(ctx_->stream, h.desc));
         v.cbase = track(dev_upload(ctx_->stream, h.cbase));
         v.off = track(dev_upload(ctx_->stream, h.off));
-        v.c16 = track(dev_upload(ctx_->stream, h.c16));
+        if (!h.c16.empty()) v.c16 = track(dev_upload(ctx_->stream, h.c16));
+        else v.c32 = track(dev_upload(ctx_->stream, h.c32));
+        v.val = track(dev_upload(ctx_->stream, h.val));
         return v;
     }
 

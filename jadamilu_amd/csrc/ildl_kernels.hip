@@ -191,27 +191,26 @@ __global__ __launch_bounds__(kB) void k_csr(int nrows, const int *__restrict__ p
     }
 }
 
-// CSR-stream form: a block owns a run of consecutive rows
-// with at most CAP - 2 entries (and at most kB rows), or a single longer row.
-// It streams the entries of its rows (consecutive in CSR) with coalesced,
-// independent loads, parks the products in LDS, then sums each row with a
-// group of t lanes (t = the power of two that spreads the block's rows over
-// its 256 threads, at most 64) and a butterfly.  Every row is written.
+// CSR-stream form: a block owns a run of consecutive rows with at most CAP
+// entries (and at most kB rows), or a single longer row.  It streams the entries
+// of its rows with coalesced, independent loads, parks the products in LDS, then
+// sums each row with a group of t lanes (t = the power of two that spreads the
+// block's rows over its 256 threads, at most 64) and a butterfly.  Every row is
+// written.
 //
-// Bound by memory on large levels and by the chain of dependent loads on
-// small ones, so the chain is kept to three: the block's descriptor; then
-// columns, values, the row's entry range and its RowOp inputs together; then the gathers
-// of x.  A thread takes entries in pairs (16 bytes of values, 4 or 8 of
-// columns a load); pairs start at an even entry, so the first may hold an
-// entry of the block before and the last one of the block behind, which are
-// loaded (the arrays end in two spare entries) and not summed.  Columns are
-// 16-bit offsets from the block's smallest column where they span less than
-// 2^16.  Level-1 and level-2 sweeps, before (2048 entries a block, one entry a
-// load, row pointers read in two dependent steps) -> now: 128^3 Laplacian
-// (7.5M and 10.0M entries) 26.4 -> 24.7 and 27.4 -> 27.0 us, 64^3 (1.0M and
-// 1.2M) 7.2 -> 6.0 and 6.9 -> 5.4 us, Anderson L = 32 (609k) 8.1 -> 5.4 us.
-template <int CAP, typename T, typename W>
-__global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restrict__ idx,
+// Bound by memory on large levels and by the chain of dependent loads on small
+// ones, so the chain is kept to two: columns and values (at places that follow
+// from the block's number) together with the block's descriptor; then the
+// gathers of x together with the row's entry range and its RowOp inputs.  A
+// thread takes entries in pairs (16 bytes of values, 4 or 8 of columns a load).
+// From 2048 entries a block, one entry a load and row pointers in two dependent
+// steps to entries in pairs behind one descriptor: sweeps of the 128^3 Laplacian
+// (7.5M and 10.0M entries) 26.4 -> 24.7 and 27.4 -> 27.0 us, of 64^3 (1.0M and
+// 1.2M) 7.2 -> 6.0 and 6.9 -> 5.4 us, of Anderson L = 32 (609k) 8.1 -> 5.4 us; to
+// places that need no descriptor: a 64^3 apply 250 -> 244 us, a 73x61x51 solve
+// 72.6 -> 70.3 ms, a 128^3 solve 951 -> 925 ms.
+template <int CAP, bool NARROW, typename T, typename W>
+__global__ __launch_bounds__(kB) void k_stream(StreamView<T> M, const int *__restrict__ idx,
                                                const T *__restrict__ val, const W *x,
                                                RowOp<W> op, int xcd) {
     typedef T T2 __attribute__((ext_vector_type(2)));
@@ -221,11 +220,26 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restri
     static_assert(kPairs * kB * 2 == CAP, "a block holds kPairs pairs per thread");
     const long blk = logical_block(xcd);
     const int tid = threadIdx.x;
+    int c0[kPairs], c1[kPairs];
+    T2 v[kPairs];
+#pragma unroll
+    for (int u = 0; u < kPairs; ++u) {
+        const long k = blk * (CAP / 2) + tid + u * kB;
+        if (NARROW) {
+            const ushort2 q = ((const ushort2 *)M.c16)[k];
+            c0[u] = q.x;
+            c1[u] = q.y;
+        } else {
+            const int2 q = ((const int2 *)M.c32)[k];
+            c0[u] = q.x;
+            c1[u] = q.y;
+        }
+        v[u] = ((const T2 *)M.val)[k];
+    }
     const int4 d = M.desc[blk];
-    const int cb = M.cbase[blk];
-    const int r0 = d.x, nr = d.y & 0xffff, e0 = d.z, ne = d.w;
-    const bool narrow = d.y >> 16;
-    if (ne > CAP - 2) {  // one long row
+    const int cb = NARROW ? M.cbase[blk] : 0;
+    const int r0 = d.x, nr = d.y, e0 = d.z, ne = d.w;
+    if (ne > CAP) {  // one long row
         double s0 = 0.0, s1 = 0.0;
         int k = e0 + tid;
         for (; k + kB < e0 + ne; k += 2 * kB) {
@@ -260,53 +274,21 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView M, const int *__restri
         b = o[1];
         if (l == 0) in.load(op, r0 + g);
     }
-    const int ea = e0 & ~1, sh = e0 & 1, tot = ne + sh;  // entries from the even start on
-    if (ne > 0) {
-        const int last = (tot + 1) / 2 - 1;
-        int c0[kPairs], c1[kPairs];
-        T v0[kPairs], v1[kPairs];
-        if (narrow) {
-            const ushort2 *c = (const ushort2 *)(M.c16 + ea);
+    // padding has column 0 of the block (a valid place) and is not summed
 #pragma unroll
-            for (int u = 0; u < kPairs; ++u) {
-                const ushort2 q = c[min(tid + u * kB, last)];
-                c0[u] = cb + q.x;
-                c1[u] = cb + q.y;
-            }
-        } else {
-            const int2 *c = (const int2 *)(idx + ea);
-#pragma unroll
-            for (int u = 0; u < kPairs; ++u) {
-                const int2 q = c[min(tid + u * kB, last)];
-                c0[u] = q.x;
-                c1[u] = q.y;
-            }
-        }
-        const T2 *v = (const T2 *)(val + ea);
-#pragma unroll
-        for (int u = 0; u < kPairs; ++u) {
-            const T2 q = v[min(tid + u * kB, last)];
-            v0[u] = q.x;
-            v1[u] = q.y;
-        }
-#pragma unroll
-        for (int u = 0; u < kPairs; ++u) {
-            // threads past the end repeat the last pair; an entry that is not
-            // the block's own takes its partner's column (a narrow offset
-            // holds from its own block's base only)
-            const int k = 2 * min(tid + u * kB, last);
-            if (k < sh) c0[u] = c1[u];
-            if (k + 1 >= tot) c1[u] = c0[u];
+    for (int u = 0; u < kPairs; ++u) {
+        const int k = 2 * (tid + u * kB);
+        if (k < ne) {
             double2 p;
-            p.x = (double)v0[u] * (double)x[c0[u]];
-            p.y = (double)v1[u] * (double)x[c1[u]];
-            if (tid + u * kB <= last) *(double2 *)(prod + k) = p;
+            p.x = (double)v[u].x * (double)x[cb + c0[u]];
+            p.y = (double)v[u].y * (double)x[cb + c1[u]];
+            *(double2 *)(prod + k) = p;
         }
     }
     __syncthreads();
     double s = 0.0;
     if (mine)
-        for (int k = sh + a + l; k < sh + b; k += t) s += prod[k];
+        for (int k = a + l; k < b; k += t) s += prod[k];
     for (int o = t / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, t);
     if (mine && l == 0) in.store(op, r0 + g, s);
 }
@@ -405,11 +387,18 @@ void ildl_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx, 
 #undef JDHIP_C
 }
 template <typename T, typename W>
-void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
+void ildl_stream(const Put &s, const StreamView<T> &M, const int *idx, const T *val, const W *x,
                  const RowOp<W> &op, int xcd) {
     if (M.nblk <= 0) return;
-    if (M.cap == 512) put(s, k_stream<512, T, W>, M.nblk, M, idx, val, x, op, xcd);
-    else put(s, k_stream<1024, T, W>, M.nblk, M, idx, val, x, op, xcd);
+#define JDHIP_ST(C, N) put(s, k_stream<C, N, T, W>, M.nblk, M, idx, val, x, op, xcd)
+    if (M.c16) {
+        if (M.cap == 512) JDHIP_ST(512, true);
+        else JDHIP_ST(1024, true);
+    } else {
+        if (M.cap == 512) JDHIP_ST(512, false);
+        else JDHIP_ST(1024, false);
+    }
+#undef JDHIP_ST
 }
 
 // Entries a block holds: 1024 where that leaves enough blocks for the 256 CUs,
@@ -417,35 +406,52 @@ void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val
 // 609k 5.4 / 5.8, 988k 6.3 / 6.0, 1.2M 5.8 / 5.4, 7.5M 28.7 / 24.7.
 static constexpr long kStreamWide = 800000;
 
-StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx) {
-    StreamHost h;
+template <typename T>
+StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx,
+                           const std::vector<T> &val) {
+    StreamHost<T> h;
     const int nnz = ptr[nrows];
     h.cap = nnz >= kStreamWide ? 1024 : 512;
-    const int most = h.cap - 2;  // a block may start one entry before its own
-    h.c16.assign((size_t)nnz + kStreamPad, 0);
+    bool narrow = true;
     int r = 0;
     while (r < nrows) {
         const int r0 = r, e0 = ptr[r];
-        while (r < nrows && r - r0 < kB && ptr[r + 1] - e0 <= most) ++r;
+        while (r < nrows && r - r0 < kB && ptr[r + 1] - e0 <= h.cap) ++r;
         if (r == r0) ++r;  // a long row alone
         const int ne = ptr[r] - e0;
         int cmin = INT_MAX, cmax = INT_MIN;
-        for (int k = e0; k < e0 + ne; ++k) {
-            cmin = std::min(cmin, idx[k]);
-            cmax = std::max(cmax, idx[k]);
-        }
+        if (ne <= h.cap)
+            for (int k = e0; k < e0 + ne; ++k) {
+                cmin = std::min(cmin, idx[k]);
+                cmax = std::max(cmax, idx[k]);
+            }
         if (cmin > cmax) cmin = cmax = 0;
-        const bool narrow = (long)cmax - cmin < 65536;
-        if (narrow)
-            for (int k = e0; k < e0 + ne; ++k) h.c16[k] = (unsigned short)(idx[k] - cmin);
-        h.desc.push_back(make_int4(r0, (r - r0) | (narrow ? 1 << 16 : 0), e0, ne));
-        h.cbase.push_back(narrow ? cmin : 0);
+        narrow = narrow && (long)cmax - cmin < 65536;
+        h.desc.push_back(make_int4(r0, r - r0, e0, ne));
+        h.cbase.push_back(cmin);
         // entry range of each row, from the block's first entry (a long row's
         // range is not read)
         for (int i = r0; i <= r; ++i) h.off.push_back((unsigned short)(ptr[i] - e0));
     }
+    const size_t slots = h.desc.size() * h.cap;
+    h.val.assign(slots, T(0));
+    if (narrow) h.c16.assign(slots, 0);
+    else h.c32.assign(slots, 0);
+    for (size_t b = 0; b < h.desc.size(); ++b) {
+        const int e0 = h.desc[b].z, ne = h.desc[b].w;
+        if (ne > h.cap) continue;
+        std::copy(val.begin() + e0, val.begin() + e0 + ne, h.val.begin() + b * h.cap);
+        for (int k = 0; k < ne; ++k) {
+            if (narrow) h.c16[b * h.cap + k] = (unsigned short)(idx[e0 + k] - h.cbase[b]);
+            else h.c32[b * h.cap + k] = idx[e0 + k];
+        }
+    }
     return h;
 }
+template StreamHost<double> build_stream(int, const std::vector<int> &, const std::vector<int> &,
+                                         const std::vector<double> &);
+template StreamHost<float> build_stream(int, const std::vector<int> &, const std::vector<int> &,
+                                        const std::vector<float> &);
 
 template <typename W>
 void ildl_dscale(const Put &s, int n, const double *dinv, W *x) {
@@ -497,7 +503,7 @@ void ildl_dense_gemv(const Put &s, int m, const T *Minv, const W *x, W *y) {
     template void ildl_csr<T, W>(const Put &, int, int, const int *, const int *, const T *,  \
                                  const W *, const RowOp<W> &, int);                           \
     template void ildl_dense_gemv<T, W>(const Put &, int, const T *, const W *, W *);         \
-    template void ildl_stream<T, W>(const Put &, const StreamView &, const int *, const T *,  \
+    template void ildl_stream<T, W>(const Put &, const StreamView<T> &, const int *, const T *,  \
                                     const W *, const RowOp<W> &, int);
 INST(double, double)
 INST(float, double)

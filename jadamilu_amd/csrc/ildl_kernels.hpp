@@ -82,32 +82,39 @@ void ildl_sell(const Put &s, const SellView &M, const T *val, const W *x, const 
 template <typename T, typename W>
 void ildl_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx, const T *val,
               const W *x, const RowOp<W> &op, int xcd);
-// CSR-stream form: blocks of consecutive rows with at most cap - 2 entries
-// (and 256 rows) each, or one longer row, streamed through LDS with coalesced
-// loads.  The product reads the CSR's own values and columns (which end in
-// kStreamPad spare entries, allocated and zero) beside this view:
-// desc[b] = {first row, rows + 2^16 when narrow, first entry, entries};
-// cbase[b] + c16[entry] is a narrow block's column; off[row + b] and the next
-// are a row's entry range from the block's first entry.
-constexpr int kStreamPad = 2;
+// CSR-stream form: blocks of consecutive rows with at most cap entries (and 256
+// rows) each, or one longer row, streamed through LDS with coalesced loads.
+// Block b's entries are laid out again from entry b*cap on (padded with zeros),
+// so that a block finds them without looking anything up: values val, and
+// columns c16 (offsets from cbase[b]) if every block's span less than 2^16, else
+// c32.  desc[b] = {first row, rows, first entry in the CSR, entries} (a longer
+// row is read from there); off[row + b] and the next are a row's entry range
+// from the block's first entry.
+template <typename T>
 struct StreamView {
     int nblk = 0;
     int cap = 1024;
     const int4 *desc = nullptr;
     const int *cbase = nullptr;
     const unsigned short *off = nullptr;
-    const unsigned short *c16 = nullptr;
+    const unsigned short *c16 = nullptr;  // or
+    const int *c32 = nullptr;
+    const T *val = nullptr;
 };
+template <typename T>
 struct StreamHost {
     int cap = 1024;
     std::vector<int4> desc;
-    std::vector<int> cbase;
+    std::vector<int> cbase, c32;
     std::vector<unsigned short> off, c16;
+    std::vector<T> val;
 };
-StreamHost build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx);
+template <typename T>
+StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx,
+                           const std::vector<T> &val);
 // xcd != 0: every XCD takes one contiguous range of row blocks.
 template <typename T, typename W>
-void ildl_stream(const Put &s, const StreamView &M, const int *idx, const T *val, const W *x,
+void ildl_stream(const Put &s, const StreamView<T> &M, const int *idx, const T *val, const W *x,
                  const RowOp<W> &op, int xcd);
 template <typename W>
 void ildl_dscale(const Put &s, int n, const double *dinv, W *x);

@@ -54,7 +54,7 @@ def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=3
     ctx.close()
 
 
-# rows around the 510 entries that a block of the small CSR-stream form holds
+# rows around the 512 entries that a block of the small CSR-stream form holds
 @pytest.mark.parametrize("k", [508, 509, 510, 511, 512, 513])
 @pytest.mark.parametrize("single", [False, True])
 def test_stream_rows_at_the_block_size(k, single):
@@ -76,7 +76,7 @@ def test_fused_ends_of_the_sweeps(gen, spd, sweeps, form, coupling, graph):
                single=single, spd=spd, dense_max=50)
 
 
-# a level large enough for the blocks of 1022 entries
+# a level large enough for the blocks of 1024 entries
 def test_stream_wide_blocks():
     _check(lambda: M.laplace((64, 63, 61)), {"ildl_form": 1}, 2)
 
