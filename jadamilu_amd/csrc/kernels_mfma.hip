@@ -221,20 +221,41 @@ int tall_gemm_mfma(hipStream_t s, const double *V, long ldv, int K, const double
     const long ntiles = (n + 15) / 16;
     const int g = (int)std::max<long>(1, std::min<long>(2048, (ntiles + 3) / 4));
     const int KS = (K + 3) / 4, JT = (J + 15) / 16;
+    // One kernel for each number of 4-column steps.  With K rounded up to 2,
+    // 4, 8, 12 or 16 steps the idle ones (nothing loaded, products with
+    // zeros) cost more than their share: n = 1,000,000, 24 -> 20 columns in 8
+    // steps 111 us, in 6 steps 66 (5.3 TB/s); 37 -> 18 columns in 12 steps
+    // 164, in 10 steps 83; n = 2,097,152, 20 -> 10 columns 117 -> 94, 10 -> 5
+    // columns 61 -> 46.  Loading the next tile ahead changes nothing (94),
+    // and neither does another LDS stride (Q stays in registers over the
+    // tiles).
 #define JDHIP_TG(ks, jt) \
     k_tall_gemm_mfma<ks, jt><<<g, kGB, 0, s>>>(V, ldv, K, Q, ldq, J, Y, ldy, n)
-#define JDHIP_TG_J(ks)                \
-    do {                              \
-        if (JT == 1) JDHIP_TG(ks, 1);   \
+#define JDHIP_TG_J(ks)                     \
+    case ks:                               \
+        if (JT == 1) JDHIP_TG(ks, 1);      \
         else if (JT == 2) JDHIP_TG(ks, 2); \
         else if (JT == 3) JDHIP_TG(ks, 3); \
-        else JDHIP_TG(ks, 4);            \
-    } while (0)
-    if (KS <= 2) JDHIP_TG_J(2);
-    else if (KS <= 4) JDHIP_TG_J(4);
-    else if (KS <= 8) JDHIP_TG_J(8);
-    else if (KS <= 12) JDHIP_TG_J(12);
-    else JDHIP_TG_J(16);
+        else JDHIP_TG(ks, 4);              \
+        break
+    switch (KS) {
+        JDHIP_TG_J(1);
+        JDHIP_TG_J(2);
+        JDHIP_TG_J(3);
+        JDHIP_TG_J(4);
+        JDHIP_TG_J(5);
+        JDHIP_TG_J(6);
+        JDHIP_TG_J(7);
+        JDHIP_TG_J(8);
+        JDHIP_TG_J(9);
+        JDHIP_TG_J(10);
+        JDHIP_TG_J(11);
+        JDHIP_TG_J(12);
+        JDHIP_TG_J(13);
+        JDHIP_TG_J(14);
+        JDHIP_TG_J(15);
+        JDHIP_TG_J(16);
+    }
 #undef JDHIP_TG_J
 #undef JDHIP_TG
     return 0;
