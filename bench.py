@@ -97,9 +97,12 @@ def norm1(ia, ja, a):
     return float(s.max())
 
 
-def spmv_bytes(n, nnz_u, s=8):
-    """Algorithmic bytes of one symmetric upper-CSR SpMV:
-    (s+4)*nnz_u + 4*(n+1) + 2*s*n."""
+def spmv_bytes(n, nnz_u, s=8, lanes=None):
+    """Algorithmic bytes of one symmetric SpMV: upper CSR,
+    (s+4)*nnz_u + 4*(n+1) + 2*s*n; the diagonal form (lanes -2) reads no
+    column indices and no row pointers, s*nnz_u + 2*s*n."""
+    if lanes == -2:
+        return s * nnz_u + 2 * s * n
     return (s + 4) * nnz_u + 4 * (n + 1) + 2 * s * n
 
 
@@ -149,7 +152,8 @@ def kernel_probe(ctx, n, nnz_u, reps, dev, torch, sweep=None):
     c1.record()
     c1.synchronize()
     copy_ms = c0.elapsed_time(c1) / reps
-    out.update({"spmv_avg_ms": spmv_ms, "spmv_alg_bytes": spmv_bytes(n, nnz_u),
+    out.update({"spmv_avg_ms": spmv_ms,
+                "spmv_alg_bytes": spmv_bytes(n, nnz_u, 8, ctx.stats().get("spmv_lanes")),
                 "copy_avg_ms": copy_ms, "copy_bytes_each_way": 1 << 28,
                 "copy_GBps_read_plus_write": 2 * (1 << 28) / (copy_ms * 1e-3) / 1e9})
     # the dense contractions of the outer iteration on the FP64 matrix cores,
@@ -663,7 +667,7 @@ def main():
     e1.record(stream)
     e1.synchronize()
     spmv_ms = e0.elapsed_time(e1) / args.spmv_reps
-    alg = spmv_bytes(n, nnz_u, 8)
+    alg = spmv_bytes(n, nnz_u, 8, r.stats.get("spmv_lanes"))
     achieved = alg / (spmv_ms * 1e-3) / 1e9
     traffic = {}
     tfile = os.path.join(ROOT, "profiles", f"traffic_{args.workload}.json")
