@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "../../include/jadamilu_amd.h"
+#include "reduce.hpp"
 #include "xcd.hpp"
 
 namespace jdhip {
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(kAB) void k_adjoint_csr(int n, const int *__restric
         int *cw = cols[threadIdx.x >> 6];
         double *gw = grad[threadIdx.x >> 6];
         for (int t = lane; t < total; t += 64) cw[t] = ja[first + t] - 1;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         const long ii = min(i, (long)n - 1);
         double xi[NC];
 #pragma unroll
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(kAB) void k_adjoint_csr(int n, const int *__restric
                 if (c < k) s += w.w[c] * xi[c] * xj[c];
             if (mine) gw[b - first + t] = (j == i) ? s : 2.0 * s;
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         for (int t = lane; t < total; t += 64) g[first + t] = gw[t];
         return;
     }

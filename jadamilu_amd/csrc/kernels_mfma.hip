@@ -19,6 +19,7 @@
 // D(4*r + l/16, l%16) in accumulator element r = 0..3 (measured on gfx950
 // with one-hot operands for every lane pair).
 #include "kernels.hpp"
+#include "reduce.hpp"
 
 namespace jdhip {
 
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(kGB) void k_tall_gemm_mfma(const double *__restrict
             // D(4*r + lk, li) -> ys[col li][row]
 #pragma unroll
             for (int r = 0; r < 4; ++r) ys[wave][li * 17 + 4 * r + lk] = acc[r];
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             // 4 columns per pass, 16 contiguous rows each
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(kGB) void k_tall_gemm_mfma(const double *__restrict
                 const int j = tj * 16 + c;
                 if (j < J && r0 + li < n) Y[(long)j * ldy + r0 + li] = ys[wave][c * 17 + li];
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
         }
     }
 }

@@ -11,6 +11,16 @@
 
 namespace jdhip {
 
+// Between a wave's writes to LDS and its lanes' reads of what other lanes
+// wrote: the barrier alone keeps the lanes together, but the compiler may move
+// memory accesses across it.  The fences cost nothing here (LDS serves a wave
+// in order; no instruction is added).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

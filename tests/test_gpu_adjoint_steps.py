@@ -1,5 +1,6 @@
 """The gradient kernels at every number of vectors where the count of loads in
-flight changes, on rows of 0, 1 and many entries, against the formula in NumPy.
+flight changes, on rows of 0 to 9 entries and at the limits of row length and
+entries of a wave, against the formula in NumPy.
 
 Both sides form the same products in double, at most 64 of them in a sum: they
 agree to 64 * 2^-52 of the sum of absolute terms.
@@ -13,16 +14,9 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 12, 13, 16, 17, 33, 64])
-@pytest.mark.parametrize("n", [1, 63, 65, 1500])
-def test_gradients_at_every_step(n, k):
+def _check(rows, n, k, rng):
+    """Both gradients for the rows' columns (0-based, upper triangle)."""
     from jadamilu_amd import lib
-    if not torch.cuda.is_available():
-        pytest.skip("no HIP device")
-    rng = np.random.default_rng(n + k)
-    rows = [np.unique(np.append(rng.integers(i, n, i % 9), i)) if i % 7 else np.array([], int)
-            for i in range(n)]
-    rows[n - 1] = np.array([n - 1])
     ia = np.concatenate([[1], 1 + np.cumsum([r.size for r in rows])]).astype(np.int32)
     ja = (np.concatenate(rows) + 1).astype(np.int32)
     ldx = n + 3
@@ -42,3 +36,40 @@ def test_gradients_at_every_step(n, k):
     assert (np.abs(g.cpu().numpy() - c * t.sum(0)) <= 64 * 2.0 ** -52 * c * np.abs(t).sum(0)).all()
     t = w[:, None] * X[:, :n] ** 2
     assert (np.abs(d.cpu().numpy() - t.sum(0)) <= 64 * 2.0 ** -52 * np.abs(t).sum(0)).all()
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 12, 13, 16, 17, 33, 64])
+@pytest.mark.parametrize("n", [1, 63, 65, 1500])
+def test_gradients_at_every_step(n, k):
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    rng = np.random.default_rng(n + k)
+    rows = [np.unique(np.append(rng.integers(i, n, i % 9), i)) if i % 7 else np.array([], int)
+            for i in range(n)]
+    rows[n - 1] = np.array([n - 1])
+    _check(rows, n, k, rng)
+
+
+# Row lengths of three waves of 64 rows and a partial one, at the limits up to
+# which a wave gives each lane a row (16 entries a row, 512 in its 64 rows): all
+# at a limit, one entry over it, a long row among short ones, and waves that
+# decide differently side by side.
+LENGTHS = {
+    "row 16": [16] + [0] * 63, "row 17": [17] + [0] * 63,
+    "wave 512": [8] * 64, "wave 513": [8] * 63 + [9],
+    "wave 512 of 16": [16] * 32 + [0] * 32, "wave 513 of 16": [16] * 32 + [1] + [0] * 31,
+    "long row": [3] * 40 + [150] + [0] * 23, "empty": [0] * 64,
+}
+
+
+@pytest.mark.parametrize("k", [1, 3, 10, 16, 17])
+@pytest.mark.parametrize("name", list(LENGTHS))
+@pytest.mark.parametrize("tail", [1, 41, 64])
+def test_gradients_at_the_limits_of_a_wave(name, tail, k):
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    lengths = [5] * 64 + LENGTHS[name] + [12] * 64 + LENGTHS[name][-tail:]
+    n = len(lengths)
+    rng = np.random.default_rng(k)
+    # (any columns: the kernel does not ask for the upper triangle)
+    _check([np.sort(rng.choice(n, m, replace=False)) for m in lengths], n, k, rng)
