@@ -18,7 +18,12 @@ constexpr int kMaxCols = 64;     // max columns of a tall-skinny product
 constexpr int kMaxRedBlocks = 4096;  // enough waves in flight to cover HBM latency
 constexpr int kMaxPartials = kMaxRedBlocks * 64;  // reduction scratch (doubles)
 // Blocks of an inner-step kernel: every block of the next kernel sums their
-// partial sums again, so there are few of them
+// partial sums again, so there are few of them.  Two a CU are enough where a
+// thread's loads are all in flight: k_multidot of 8 columns takes 37.8 us with
+// 512 blocks, 38.5 with 1,024 and 40.4 with 4,096 (3,000,000 rows; 14.5 / 14.9 /
+// 21.2 for 1,000,000), of one column 11.3 / 9.2 / 9.7; against 4,096 blocks and
+// finishing launches of their own, k_cg_update 24.0 against 22.8 + 4.7 us,
+// k_project_rho of 4 columns 26.5 against 24.9 + 4.3.
 constexpr int kInnerBlocks = 512;
 constexpr int kInnerPartials = kInnerBlocks * (kMaxCols + 8);
 
