@@ -296,7 +296,7 @@ int jdhip_pjd_batch_opts(int device, int nitems, jdhip_batch_item *items, int nw
 /* ---- symmetric SpMV (MATVECA, JDaux.F:3397-3418) ------------------------- */
 /* Upload a 1-based upper-triangle CSR (diagonal anywhere in each row) as the
  * device operator of ctx; 0 on success.  lanes_per_row: 0 = chosen (for
- * at least 4,096 rows on at most 16 upper diagonals, one array per diagonal of
+ * at least 4,096 rows on at most 7 upper diagonals, one array per diagonal of
  * the upper triangle; else the formats below timed on this matrix), -1 = sliced ELL (64-row slices, one
  * lane per row, 16-bit column offsets where a slice allows), k > 0 = CSR with
  * k lanes per row. */

@@ -95,7 +95,12 @@ void argmax_abs(hipStream_t s, const RedBuf &rb, const double *x, long n, double
 // diagonal, val[k*stride + i] = A(i, i + off[k]), off ascending from 0; for
 // slice s of 64 rows and diagonal k, mask[2*(s*nd + k)] has the rows with an
 // entry A(i, i + off[k]) and the next word those with A(i, i - off[k]).
-constexpr int kDiaMax = 16;  // most diagonals of the upper triangle
+// Most diagonals of the upper triangle: the kernels have a row's entries all in
+// flight at once, in registers, up to this many.  A loop over more (8 to 16) was
+// slower than the general formats up to 250,000 rows (27-point stencil of 40^3:
+// SpMV 4.5 -> 7.2 us; 5,000 rows on 16 diagonals 2.3 -> 7.6) and with several
+// vectors beyond (three on 80^3 36.8 -> 60.2), and took longer to set up.
+constexpr int kDiaMax = 7;
 // most rows: byte offsets of 32 bits, and a partial sum of u.y per 256 rows
 constexpr int kDiaRows = kMaxPartials * 256;
 struct DiaDev {
@@ -104,12 +109,12 @@ struct DiaDev {
     double *val = nullptr;
     float *valf = nullptr;  // FP32 copy
     unsigned long long *mask = nullptr;
-    long off[kDiaMax] = {};
+    int off[kDiaMax] = {};
 };
 struct DiaHost {
     int nd = 0, nslices = 0;
     long stride = 0;
-    std::vector<long> off;
+    std::vector<int> off;
     std::vector<double> val;
     std::vector<unsigned long long> mask;
 };

@@ -51,7 +51,7 @@ __device__ __forceinline__ T at(const T *p, unsigned i) {
     const unsigned row = (unsigned)(sl * 64 + lane)
 
 // Entries below the diagonal in ascending column order, then the diagonal and
-// above: the order of a row's entries in the CSR copy.  ND > 0: the number of
+// above: the order of a row's entries in the CSR copy.  ND: the number of
 // diagonals, all loads issued before the first use.
 template <typename T, typename TA, int ND, bool ETA, bool UDOT>
 __global__ __launch_bounds__(kBlock) void k_spmv_dia(DiaDev A, const TA *__restrict__ val,
@@ -63,45 +63,28 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dia(DiaDev A, const TA *__restr
     if (sl < A.nslices && row < (unsigned)A.n) {
         const u64 *m = A.mask + sl * 2 * A.nd;
         double s = 0.0;
-        if constexpr (ND > 0) {
-            double vu[ND], vl[ND];
-            T xu[ND], xl[ND];
+        double vu[ND], vl[ND];
+        T xu[ND], xl[ND];
 #pragma unroll
-            for (int k = 0; k < ND; ++k) {
-                const u64 mu = m[2 * k], ml = m[2 * k + 1];
-                const unsigned d = (unsigned)A.off[k];
-                vu[k] = vl[k] = 0.0;
-                xu[k] = xl[k] = T(0);
-                if (mu) {
-                    vu[k] = (double)at(val + k * A.stride, row);
-                    xu[k] = at(x, has(mu) ? row + d : row);
-                }
-                if (k > 0 && ml) {
-                    const unsigned j = has(ml) ? row - d : row;
-                    vl[k] = (double)at(val + k * A.stride, j);
-                    xl[k] = at(x, j);
-                }
+        for (int k = 0; k < ND; ++k) {
+            const u64 mu = m[2 * k], ml = m[2 * k + 1];
+            const unsigned d = (unsigned)A.off[k];
+            vu[k] = vl[k] = 0.0;
+            xu[k] = xl[k] = T(0);
+            if (mu) {
+                vu[k] = (double)at(val + k * A.stride, row);
+                xu[k] = at(x, has(mu) ? row + d : row);
             }
-#pragma unroll
-            for (int k = ND - 1; k > 0; --k) s = has(m[2 * k + 1]) ? s + vl[k] * (double)xl[k] : s;
-#pragma unroll
-            for (int k = 0; k < ND; ++k) s = has(m[2 * k]) ? s + vu[k] * (double)xu[k] : s;
-        } else {
-            for (int k = A.nd - 1; k > 0; --k) {
-                const u64 ml = m[2 * k + 1];
-                if (!ml) continue;
-                const unsigned j = has(ml) ? row - (unsigned)A.off[k] : row;
-                const double v = (double)at(val + k * A.stride, j), xj = (double)at(x, j);
-                s = has(ml) ? s + v * xj : s;
-            }
-            for (int k = 0; k < A.nd; ++k) {
-                const u64 mu = m[2 * k];
-                if (!mu) continue;
-                const double v = (double)at(val + k * A.stride, row);
-                const double xj = (double)at(x, has(mu) ? row + (unsigned)A.off[k] : row);
-                s = has(mu) ? s + v * xj : s;
+            if (k > 0 && ml) {
+                const unsigned j = has(ml) ? row - d : row;
+                vl[k] = (double)at(val + k * A.stride, j);
+                xl[k] = at(x, j);
             }
         }
+#pragma unroll
+        for (int k = ND - 1; k > 0; --k) s = has(m[2 * k + 1]) ? s + vl[k] * (double)xl[k] : s;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) s = has(m[2 * k]) ? s + vu[k] * (double)xu[k] : s;
         if (ETA) s -= eta * (double)x[row];
         const T yi = (T)s;
         y[row] = yi;
@@ -110,11 +93,10 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dia(DiaDev A, const TA *__restr
     if (UDOT) grid_reduce<1>(acc, 1, partials, 0, nullptr);
 }
 
-// kv vectors.  ND > 0: a row's values are loaded once and stay in registers for
-// all of them; the vectors go by one at a time (two or four at a time, whose
-// loads would all be in flight, leave too few waves: 78 and 88 us against 70
-// for 5 vectors of the 128^3 Laplacian).  ND = 0: any number of diagonals,
-// eight vectors at a time.
+// kv vectors.  A row's values are loaded once and stay in registers for all of
+// them; the vectors go by one at a time (two or four at a time, whose loads
+// would all be in flight, leave too few waves: 78 and 88 us against 70 for 5
+// vectors of the 128^3 Laplacian).
 template <int ND>
 __global__ __launch_bounds__(kBlock) void k_spmm_dia(DiaDev A, int kv,
                                                      const double *__restrict__ x, long ldx,
@@ -122,59 +104,33 @@ __global__ __launch_bounds__(kBlock) void k_spmm_dia(DiaDev A, int kv,
     JDHIP_SLICES(sl, row);
     if (sl >= A.nslices || row >= (unsigned)A.n) return;
     const u64 *m = A.mask + sl * 2 * A.nd;
-    if constexpr (ND > 0) {
-        double vu[ND], vl[ND];
-        unsigned ju[ND], jl[ND];
+    double vu[ND], vl[ND];
+    unsigned ju[ND], jl[ND];
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        const unsigned d = (unsigned)A.off[k];
+        vu[k] = vl[k] = 0.0;
+        ju[k] = has(m[2 * k]) ? row + d : row;
+        jl[k] = has(m[2 * k + 1]) ? row - d : row;
+        if (m[2 * k]) vu[k] = at(A.val + k * A.stride, row);
+        if (k > 0 && m[2 * k + 1]) vl[k] = at(A.val + k * A.stride, jl[k]);
+    }
+#pragma unroll 1
+    for (int c = 0; c < kv; ++c) {
+        const double *xc = x + c * ldx;
+        double xu[ND], xl[ND];
 #pragma unroll
         for (int k = 0; k < ND; ++k) {
-            const unsigned d = (unsigned)A.off[k];
-            vu[k] = vl[k] = 0.0;
-            ju[k] = has(m[2 * k]) ? row + d : row;
-            jl[k] = has(m[2 * k + 1]) ? row - d : row;
-            if (m[2 * k]) vu[k] = at(A.val + k * A.stride, row);
-            if (k > 0 && m[2 * k + 1]) vl[k] = at(A.val + k * A.stride, jl[k]);
+            xu[k] = xl[k] = 0.0;
+            if (m[2 * k]) xu[k] = at(xc, ju[k]);
+            if (k > 0 && m[2 * k + 1]) xl[k] = at(xc, jl[k]);
         }
-#pragma unroll 1
-        for (int c = 0; c < kv; ++c) {
-            const double *xc = x + c * ldx;
-            double xu[ND], xl[ND];
+        double s = 0.0;
 #pragma unroll
-            for (int k = 0; k < ND; ++k) {
-                xu[k] = xl[k] = 0.0;
-                if (m[2 * k]) xu[k] = at(xc, ju[k]);
-                if (k > 0 && m[2 * k + 1]) xl[k] = at(xc, jl[k]);
-            }
-            double s = 0.0;
+        for (int k = ND - 1; k > 0; --k) s = has(m[2 * k + 1]) ? s + vl[k] * xl[k] : s;
 #pragma unroll
-            for (int k = ND - 1; k > 0; --k) s = has(m[2 * k + 1]) ? s + vl[k] * xl[k] : s;
-#pragma unroll
-            for (int k = 0; k < ND; ++k) s = has(m[2 * k]) ? s + vu[k] * xu[k] : s;
-            y[row + c * ldy] = s;
-        }
-    } else {
-        constexpr int G = 8;
-        for (int c0 = 0; c0 < kv; c0 += G) {
-            double s[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) s[g] = 0.0;
-            auto diagonal = [&](u64 mk, unsigned jv, unsigned jx, int k) {
-                const double v = at(A.val + k * A.stride, has(mk) ? jv : row);
-                const unsigned j = has(mk) ? jx : row;
-                double t[G];
-#pragma unroll
-                for (int g = 0; g < G; ++g) t[g] = at(x + (long)min(c0 + g, kv - 1) * ldx, j);
-#pragma unroll
-                for (int g = 0; g < G; ++g) s[g] = has(mk) ? s[g] + v * t[g] : s[g];
-            };
-            for (int k = A.nd - 1; k > 0; --k)
-                if (m[2 * k + 1])
-                    diagonal(m[2 * k + 1], row - (unsigned)A.off[k], row - (unsigned)A.off[k], k);
-            for (int k = 0; k < A.nd; ++k)
-                if (m[2 * k]) diagonal(m[2 * k], row, row + (unsigned)A.off[k], k);
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-                if (c0 + g < kv) y[row + (long)(c0 + g) * ldy] = s[g];
-        }
+        for (int k = 0; k < ND; ++k) s = has(m[2 * k]) ? s + vu[k] * xu[k] : s;
+        y[row + c * ldy] = s;
     }
 }
 #undef JDHIP_SLICES
@@ -207,8 +163,7 @@ int product(hipStream_t s, const RedBuf &rb, const DiaDev &A, const TA *val, con
         case 4: JDHIP_ND(4); break;
         case 5: JDHIP_ND(5); break;
         case 6: JDHIP_ND(6); break;
-        case 7: JDHIP_ND(7); break;
-        default: JDHIP_ND(0); break;
+        default: JDHIP_ND(7); break;
     }
 #undef JDHIP_ND
     if (!u) return 0;
@@ -243,8 +198,7 @@ void spmm_dia(hipStream_t s, const DiaDev &A, int k, const double *x, long ldx, 
         case 4: JDHIP_ND(4); break;
         case 5: JDHIP_ND(5); break;
         case 6: JDHIP_ND(6); break;
-        case 7: JDHIP_ND(7); break;
-        default: JDHIP_ND(0); break;
+        default: JDHIP_ND(7); break;
 #undef JDHIP_ND
     }
 }
@@ -288,7 +242,7 @@ bool build_dia(int n, const int *ia, const int *ja, const double *a, DiaHost &h)
     std::sort(h.off.begin(), h.off.end());
     int rank[kDiaMax];
     for (int k = 0; k < nd; ++k)
-        rank[k] = (int)(std::lower_bound(h.off.begin(), h.off.end(), (long)d[k]) - h.off.begin());
+        rank[k] = (int)(std::lower_bound(h.off.begin(), h.off.end(), d[k]) - h.off.begin());
     h.val.assign((size_t)nd * h.stride, 0.0);
     h.mask.assign((size_t)h.nslices * 2 * nd, 0);
     for (int i = 0; i < n; ++i)

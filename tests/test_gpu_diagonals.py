@@ -88,8 +88,9 @@ def _sparse_diagonals(n):
     (lambda: M.from_pairs(5000, np.zeros(0, int), np.zeros(0, int), np.zeros(0),
                           np.arange(5000.0)), True),
     (lambda: _holes(4099, 1), True),
-    (lambda: _many(5000, 7), True),
-    (lambda: _many(5000, 15), True),
+    (lambda: _many(5000, 6), True),
+    (lambda: _many(5000, 7), False),
+    (lambda: _many(5000, 15), False),
     (lambda: _many(5000, 16), False),
     (lambda: _sparse_diagonals(20000), False),
     (lambda: _twice(5000), False),
