@@ -93,12 +93,18 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dia(DiaDev A, const TA *__restr
     if (UDOT) grid_reduce<1>(acc, 1, partials, 0, nullptr);
 }
 
-// kv vectors.  A row's values are loaded once and stay in registers for all of
-// them; the vectors go by one at a time (two or four at a time, whose loads
-// would all be in flight, leave too few waves: 78 and 88 us against 70 for 5
-// vectors of the 128^3 Laplacian).
+// kv vectors, per of them a block.  A row's values are loaded once and stay in
+// registers for these; the vectors go by one at a time (two or four at a time,
+// whose loads would all be in flight, leave too few waves: 78 and 88 us against
+// 70 for 5 vectors of the 128^3 Laplacian).  A small matrix is bound by that
+// chain of loads, so its vectors go to different blocks.  Us for 3 / 10 vectors,
+// all in one block, spread, and the CSR form: 64^2 Laplacian 2.99, 2.38, 2.40 /
+// 5.22, 2.42, 5.10; 250^2 3.19, 2.90, 4.11 / 6.13, 4.75, 10.7; Anderson L = 17
+// (7 diagonals) 3.81, 2.91, 2.61 / 7.29, 2.96, 5.60.  Spread to 1,024 blocks, L =
+// 50 takes 5.36 instead of 4.94 us for 3 vectors, to 4,096 6.22.
+constexpr int kSpread = 512;
 template <int ND>
-__global__ __launch_bounds__(kBlock) void k_spmm_dia(DiaDev A, int kv,
+__global__ __launch_bounds__(kBlock) void k_spmm_dia(DiaDev A, int kv, int per,
                                                      const double *__restrict__ x, long ldx,
                                                      double *__restrict__ y, long ldy) {
     JDHIP_SLICES(sl, row);
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_dia(DiaDev A, int kv,
         if (k > 0 && m[2 * k + 1]) vl[k] = at(A.val + k * A.stride, jl[k]);
     }
 #pragma unroll 1
-    for (int c = 0; c < kv; ++c) {
+    for (int c = blockIdx.y * per; c < min(kv, (int)(blockIdx.y + 1) * per); ++c) {
         const double *xc = x + c * ldx;
         double xu[ND], xl[ND];
 #pragma unroll
@@ -190,8 +196,11 @@ void spmm_dia(hipStream_t s, const DiaDev &A, int k, const double *x, long ldx, 
               long ldy) {
     const long blocks = ((long)A.nslices + kBlock / 64 - 1) / (kBlock / 64);
     const int g = (int)blocks;
+    // vectors a block takes: all of them, or so many that there are kSpread blocks
+    const int groups = std::max(1, std::min(k, kSpread / g)), per = (k + groups - 1) / groups;
     switch (A.nd) {
-#define JDHIP_ND(D) k_spmm_dia<D><<<g, kBlock, 0, s>>>(A, k, x, ldx, y, ldy)
+#define JDHIP_ND(D) \
+    k_spmm_dia<D><<<dim3(g, (k + per - 1) / per), kBlock, 0, s>>>(A, k, per, x, ldx, y, ldy)
         case 1: JDHIP_ND(1); break;
         case 2: JDHIP_ND(2); break;
         case 3: JDHIP_ND(3); break;
