@@ -48,3 +48,11 @@ def _most_in_flight(source, kernel):
     ("k_project_rhoIdLi4E", 6), ("k_project_rhoIdLi8E", 10), ("k_project_rhoIfLi8E", 10)])
 def test_inner_step(kernel, loads):
     assert _most_in_flight("kernels_inner.hip", kernel) >= loads
+
+
+@pytest.mark.parametrize("kernel,loads", [
+    # a value and an x for every entry of a row, with one more x and u
+    ("k_spmv_diaIddLi4ELb0ELb1E", 15), ("k_spmv_diaIddLi7ELb0ELb1E", 27),
+    ("k_spmv_diaIffLi4ELb0ELb1E", 15), ("k_spmv_diaIfdLi4ELb0ELb1E", 15)])
+def test_diagonal_product(kernel, loads):
+    assert _most_in_flight("kernels_dia.hip", kernel) >= loads
