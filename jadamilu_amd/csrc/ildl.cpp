@@ -204,19 +204,28 @@ struct SellDev {
     long nnz16 = 0, nnz32 = 0;
 };
 
-// Kernel form of a product with nnz entries over rows rows before any timing:
+// Kernel form of a product (CSR row pointers ptr) before any timing:
 // CSR-stream for large products, whose entries it balances, else CSR lane
 // groups of about the average row length.  Measured (us a launch in a graph,
 // stream / the rule's lanes): 609k entries of 22 a row 5.4 / 6.2, 354k of 98
-// 3.8 / 3.9, 186k of 16 3.5 / 3.3, 107k of 134 3.8 / 3.1, 22k of 2.8 3.2 / 2.6.
+// 3.8 / 3.9, 186k of 16 3.5 / 3.3, 107k of 134 3.8 / 3.1, 22k of 2.8 3.2 / 2.6; an
+// apply of 50,000 rows of one entry, 21.8 us in stream, 31.5 with 8 lanes.
+// A row much longer than its lanes is a chain of its own (0.3 us for every four
+// entries a lane), which stream spreads over a block: an apply with rows of up
+// to 9,706 entries among short ones (30,001 rows, four levels) 427 us by the
+// average alone, 166 with the last line, which lies between 8 and 64 times the
+// lanes without a difference.
 constexpr long kTimed = 200000;
-inline int pick_form(long nnz, int rows) {
+inline int pick_form(const std::vector<int> &ptr) {
+    const int rows = (int)ptr.size() - 1;
     if (rows <= 0) return 0;
+    const long nnz = ptr[rows];
     if (nnz >= kTimed || rows >= 32768) return 1;
     const double avg = 0.8 * (double)nnz / rows;
-    int lanes = 8;
+    int lanes = 8, longest = 0;
     while (lanes < 64 && lanes < avg) lanes *= 2;
-    return lanes;
+    for (int r = 0; r < rows; ++r) longest = std::max(longest, ptr[r + 1] - ptr[r]);
+    return longest > 16 * lanes ? 1 : lanes;
 }
 
 template <typename T, typename W>
@@ -368,6 +377,8 @@ class IldlImpl : public IldlImplBase {
             D.lt_val = track(dev_upload(ctx_->stream, tv));
             D.st_b = upload_stream(nB, bp, bi, bv);
             D.st_t = upload_stream(nB, tp, ti, tv);
+            D.wf = pick_form(bp);
+            D.wb = pick_form(tp);
             D.sf = upload_sell(build_sell(nB, bp, bi, bv, sigma_));
             D.sb = upload_sell(build_sell(nB, tp, ti, tv, sigma_));
             // dependency levels from the triangular (factor) numbering
@@ -387,15 +398,14 @@ class IldlImpl : public IldlImplBase {
             D.lc_idx = track(dev_upload(ctx_->stream, ci));
             D.lc_val = track(dev_upload(ctx_->stream, cv));
             D.st_c = upload_stream(nC, cp, ci, cv);
-            D.wc = pick_form((long)ci.size(), nC);
-            D.wf = D.wb = pick_form((long)bi.size(), nB);
+            D.wc = pick_form(cp);
             transpose(nC, nB, cp, ci, cv, tp, ti, tv);
             D.sct = upload_sell(build_sell(nB, tp, ti, tv, sigma_, true));
             D.lct_ptr = track(dev_upload(ctx_->stream, tp));
             D.lct_idx = track(dev_upload(ctx_->stream, ti));
             D.lct_val = track(dev_upload(ctx_->stream, tv));
             D.st_ct = upload_stream(nB, tp, ti, tv);
-            D.wct = pick_form((long)ti.size(), nB);
+            D.wct = pick_form(tp);
             D.buf = track(dev_alloc<W>(n));
             D.out = track(dev_alloc<W>(n));
             D.t1 = track(dev_alloc<W>(std::max(nB, 1)));

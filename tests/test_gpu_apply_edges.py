@@ -26,6 +26,7 @@ def _hub(n, k):
 
 
 def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=300):
+    """The apply against the oracle's; the kernel forms chosen."""
     from jadamilu_amd.ildl import IldlFactor
     from jadamilu_amd.jd import Context
     if not torch.cuda.is_available():
@@ -51,7 +52,9 @@ def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=3
         zo = O.ildl_apply(ex, r, sweeps=sweeps)
         tol = 2e-5 if single else 1e-12
         assert np.linalg.norm(zd.cpu().numpy() - zo) <= tol * np.linalg.norm(zo)
+    forms = ctx.ildl_level_forms()
     ctx.close()
+    return forms
 
 
 # rows around the 512 entries that a block of the small CSR-stream form holds
@@ -59,6 +62,16 @@ def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=3
 @pytest.mark.parametrize("single", [False, True])
 def test_stream_rows_at_the_block_size(k, single):
     _check(lambda: _hub(700, k), {"ildl_form": 1}, 3, single=single)
+
+
+# a row of k - 1 entries of L_B, or (k = 4000) of 1,281 of the coupling block,
+# among rows of one: lane groups up to 16 times their 8 lanes, CSR-stream beyond;
+# forms of the forward and backward sweeps and of the coupling block
+@pytest.mark.parametrize("k,form", [(100, [8, 8]), (129, [8, 8]), (130, [1, 8]),
+                                    (4000, [8, 8, 1])])
+def test_long_row_among_short_ones(k, form):
+    forms = _check(lambda: _hub(4000, k), {}, 3, dense_max=0)
+    assert forms[0][:len(form)] == form
 
 
 # one, two and three sweeps: where the last sweep carries D^-1 and the addition
