@@ -349,7 +349,7 @@ int jdhip_tall_gemm(jdhip_ctx *ctx, long n, int k, int j, const double *v_dev, l
  * two solves with B per level, as the reference, the default; 1 = L_CB blocks,
  * see jdhip_ildl_coupling), "ildl_dense_max" (largest final
  * level factored densely), "spmv_lanes", "ildl_graph" (1: replay the
- * preconditioner apply from a HIP graph where it holds at most 1024 launches;
+ * preconditioner apply from a HIP graph where it holds 12 to 1024 launches;
  * 0: launch it kernel by kernel; default -1, as 1), "ildl_storage",
  * "ildl_xcd", "ildl_sigma" (device layout of the factor), "ildl_threads"
  * (host threads of the factorization), "sync_blocking" (1: the iteration's

@@ -799,8 +799,10 @@ class IldlImpl : public IldlImplBase {
         hipGraph_t g = nullptr;
         JDHIP_CHECK(hipGraphCreate(&g, 0));
         try {
-            body(Put(g));
-            JDHIP_CHECK(hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0));
+            const Put q(g);
+            body(q);
+            if (q.nodes >= kGraphMin)
+                JDHIP_CHECK(hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0));
         } catch (...) {
             hipGraphDestroy(g);
             throw;
@@ -987,8 +989,16 @@ class IldlImpl : public IldlImplBase {
 
     DevCtx *ctx_;
     IldlMultilevel<T> f_;
-    // launches that one graph holds at most (exact solves of small factors
-    // included); larger applies are bound by their kernels
+    // Launches that a graph holds.  At least: a graph launch takes the host 32 us,
+    // however few its nodes, a kernel launch 2.5-4.5 us, so short applies are
+    // enqueued one by one: a solve of 50,000 rows with 6 launches an apply takes
+    // 7.33 ms so and 8.53 ms with graphs, with 8 7.98 and 8.86, with 12 9.05 and
+    // 8.83.  (Applies alone in the stream, on two machines: of 6 launches 21.8
+    // and 33.7 us, as graphs 32.8 and 32.2; of 12 37.8 and 52.8, 39.5 and 39.7;
+    // of 24 69 and 96, 67 and 67.)  At most (exact solves, a launch per dependency
+    // level): the gain is the same for each launch (760 of them 2.72 -> 1.73 ms),
+    // but a factor of some thousand levels would hold a graph of 10^5 nodes.
+    static constexpr int kGraphMin = 12;
     static constexpr long kGraphMax = 1024;
     hipGraphExec_t graph_ = nullptr;
     bool tuning_ = false;

@@ -53,6 +53,7 @@ static void put(const Put &q, void (*k)(P...), int grid, A... args) {
                 throw std::runtime_error(std::string("HIP error ") + hipGetErrorString(e) +
                                          " adding a graph node");
             q.last = node;
+            ++q.nodes;
         },
         held);
 }

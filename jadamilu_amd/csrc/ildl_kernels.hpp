@@ -27,6 +27,7 @@ struct Put {
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     mutable hipGraphNode_t last = nullptr;
+    mutable int nodes = 0;  // in the graph so far
     Put(hipStream_t s) : stream(s) {}
     Put(hipGraph_t g) : graph(g) {}
 };
