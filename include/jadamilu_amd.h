@@ -449,13 +449,14 @@ int jdhip_ildl_level_sweeps(jdhip_ctx *ctx, int *out, int cap);
  * sweep over L_B, backward sweep over L_B^T, L_CB product, L_CB^T product):
  * 0 one lane per row on a SELL-C-sigma copy, 1 CSR-stream (row blocks of at
  * most 1024 entries staged through LDS), k >= 4 CSR with k lanes per row.
- * Chosen by timing at set-up (option ildl_autotune, default 1), else by the
- * average row length.  Fills out[0..cap-1]; returns the number of levels, or
+ * Products of at least 200,000 entries: chosen by timing at set-up (option
+ * ildl_autotune, default 1); others by their rows' lengths.  Fills out[0..cap-1]; returns the number of levels, or
  * -1 without an ILDL preconditioner.  No reference counterpart. */
 int jdhip_ildl_level_forms(jdhip_ctx *ctx, int *out, int cap);
 /* Diagnostic: time reps launches of one Jacobi sweep over the first level's
  * L_B (the largest single kernel of the preconditioner apply) on ctx's stream
- * with HIP events; *alg_bytes = its algorithmic bytes per launch.  No
+ * with HIP events; *alg_bytes = its algorithmic bytes per launch (the matrix
+ * in the kernel form chosen, without padding, and three vectors).  No
  * reference counterpart.  0 on success, -1 without an ILDL preconditioner. */
 int jdhip_ildl_time_sweep(jdhip_ctx *ctx, int reps, double *avg_ms, long *alg_bytes);
 

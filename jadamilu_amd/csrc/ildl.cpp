@@ -204,6 +204,12 @@ struct SellDev {
     long nnz16 = 0, nnz32 = 0;
 };
 
+template <typename T>
+struct StreamDev {
+    StreamView<T> v;  // device arrays of the layout
+    long nnz16 = 0, nnz32 = 0;
+};
+
 // Kernel form of a product (CSR row pointers ptr) before any timing:
 // CSR-stream for large products, whose entries it balances, else CSR lane
 // groups of about the average row length.  Measured (us a launch in a graph,
@@ -246,7 +252,7 @@ struct DevLevel {
     int *lct_ptr = nullptr, *lct_idx = nullptr;
     T *lct_val = nullptr;
     // row blocks of the CSR-stream form for L_B, L_B^T, L_CB, L_CB^T
-    StreamView<T> st_b, st_t, st_c, st_ct;
+    StreamDev<T> st_b, st_t, st_c, st_ct;
     std::vector<int> fwd_ptr, bwd_ptr;  // host level pointers
     int *fwd_rows = nullptr, *bwd_rows = nullptr;
     W *buf = nullptr, *out = nullptr, *t1 = nullptr, *t2 = nullptr;  // work vectors
@@ -489,7 +495,7 @@ class IldlImpl : public IldlImplBase {
         const int *idx = fwd ? D.lb_idx : D.lt_idx;
         const T *val = fwd ? D.lb_val : D.lt_val;
         if (form == 1) {
-            ildl_stream<T, W>(s, fwd ? D.st_b : D.st_t, idx, val, x, op, xcd_ & 1);
+            ildl_stream<T, W>(s, fwd ? D.st_b.v : D.st_t.v, idx, val, x, op, xcd_ & 1);
         } else if (form > 0) {
             ildl_csr<T, W>(s, form, D.nB, fwd ? D.lb_ptr : D.lt_ptr, idx, val, x, op, xcd_ & 1);
         } else {
@@ -508,7 +514,7 @@ class IldlImpl : public IldlImplBase {
         op.src = fresh ? nullptr : y;
         op.out = y;
         if (form == 1) {
-            ildl_stream<T, W>(s, trans ? D.st_ct : D.st_c, idx, val, x, op, xcd_ & 1);
+            ildl_stream<T, W>(s, trans ? D.st_ct.v : D.st_c.v, idx, val, x, op, xcd_ & 1);
         } else if (form > 0) {
             ildl_csr<T, W>(s, form, rows, trans ? D.lct_ptr : D.lc_ptr, idx, val, x, op,
                            xcd_ & 1);
@@ -608,10 +614,11 @@ class IldlImpl : public IldlImplBase {
         return v;
     }
 
-    StreamView<T> upload_stream(int nrows, const std::vector<int> &ptr,
-                                const std::vector<int> &idx, const std::vector<T> &val) {
+    StreamDev<T> upload_stream(int nrows, const std::vector<int> &ptr,
+                               const std::vector<int> &idx, const std::vector<T> &val) {
         const StreamHost<T> h = build_stream(nrows, ptr, idx, val);
-        StreamView<T> v;
+        StreamDev<T> d;
+        StreamView<T> &v = d.v;
         v.nblk = (int)h.desc.size();
         v.cap = h.cap;
         v.desc = track(dev_upload(ctx_->stream, h.desc));
@@ -620,7 +627,9 @@ class IldlImpl : public IldlImplBase {
         if (!h.c16.empty()) v.c16 = track(dev_upload(ctx_->stream, h.c16));
         else v.c32 = track(dev_upload(ctx_->stream, h.c32));
         v.val = track(dev_upload(ctx_->stream, h.val));
-        return v;
+        d.nnz16 = h.nnz16;
+        d.nnz32 = h.nnz32;
+        return d;
     }
 
     SellDev<T> upload_sell(const SellHost<T> &h) {
@@ -907,29 +916,37 @@ class IldlImpl : public IldlImplBase {
     void dense_data(double *minv) const override {
         for (size_t i = 0; i < f_.dinv.size(); ++i) minv[i] = (double)(T)f_.dinv[i];
     }
-    // values and column indices one product streams in the given form
-    static long mat_bytes(const SellDev<T> &M, int form, long nnz) {
-        if (form > 0) return ((long)sizeof(T) + 4) * nnz;  // CSR (lanes or stream)
-        return (long)sizeof(T) * nnz + 2 * M.nnz16 + 4 * M.nnz32;
+    // What one product with a matrix of nnz entries and rows rows streams in the
+    // given form, without padding: values, columns in the width they are read
+    // with, and what finds a row's entries.
+    static long mat_bytes(const SellDev<T> &M, const StreamDev<T> &S, int form, long nnz,
+                          long rows) {
+        const long values = (long)sizeof(T) * nnz;
+        if (form == 1)
+            return values + 2 * S.nnz16 + 4 * S.nnz32 + 2 * (rows + S.v.nblk) + 20L * S.v.nblk;
+        if (form > 0) return values + 4 * nnz + 4 * (rows + 1);
+        return values + 2 * M.nnz16 + 4 * M.nnz32 + 4 * rows;
+    }
+    long sweep_bytes(const DevLevel<T, W> &D, bool fwd) const {
+        return (fwd ? mat_bytes(D.sf, D.st_b, D.wf, D.nnz_lb, D.nB)
+                    : mat_bytes(D.sb, D.st_t, D.wb, D.nnz_lb, D.nB)) +
+               3L * (long)sizeof(W) * D.nB;
     }
     long apply_bytes() const override {
-        // per level: one pass over L_B per sweep and direction (values,
-        // indices, row map, b, x, result), L_CB and L_CB^T once,
-        // gather/scatter (perm + scal + in/out), D^-1, dense inverse.
-        // Factor values are sizeof(T) bytes, vectors sizeof(W).
-        // Matrix bytes follow each product's chosen form (int32 columns in
-        // CSR, 16- or 32-bit per SELL slice).
+        // per level: one pass over L_B per sweep and direction (matrix, b, x,
+        // result), L_CB and L_CB^T once, gather/scatter (perm + scal + in/out),
+        // D^-1, dense inverse.  Factor values are sizeof(T) bytes, vectors
+        // sizeof(W); matrix bytes follow each product's chosen form.
         const long s = sizeof(T), v = sizeof(W);
         long b = 0;
         for (const auto &D : lv_) {
             const long k = D.k > 0 ? D.k : 1;
             // F blocks: a level with a coarse part solves with B twice
             const long solves = (fform() && D.nC > 0) ? 2 : 1;
-            b += solves * (k * (mat_bytes(D.sf, D.wf, D.nnz_lb) + mat_bytes(D.sb, D.wb, D.nnz_lb)) +
-                           2 * k * (4L * D.nB + 3 * v * D.nB));
+            b += solves * k * (sweep_bytes(D, true) + sweep_bytes(D, false));
             if (solves == 2) b += v * D.nB;  // y_B, added to
-            b += mat_bytes(D.sc, D.wc, D.nnz_lc) + mat_bytes(D.sct, D.wct, D.nnz_lc) +
-                 2 * (4L * (D.nC + D.nB + 2) + v * (D.nB + D.nC));
+            b += mat_bytes(D.sc, D.st_c, D.wc, D.nnz_lc, D.nC) +
+                 mat_bytes(D.sct, D.st_ct, D.wct, D.nnz_lc, D.nB) + 2 * v * (D.nB + D.nC);
             b += 2 * (4L + v) * D.n + 2 * v * D.n + 2 * v * D.nB;
         }
         b += s * (long)f_.m * f_.m + 2 * v * f_.m;
@@ -960,9 +977,7 @@ class IldlImpl : public IldlImplBase {
         hipEventDestroy(e0);
         hipEventDestroy(e1);
         *avg_ms = ms / reps;
-        const long sz = sizeof(T);
-        (void)sz;
-        *alg_bytes = mat_bytes(D.sf, D.wf, D.nnz_lb) + 4L * D.nB + 3L * (long)sizeof(W) * D.nB;
+        *alg_bytes = sweep_bytes(D, true);
         return 0;
     }
 

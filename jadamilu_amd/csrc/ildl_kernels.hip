@@ -440,6 +440,7 @@ StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::ve
     else h.c32.assign(slots, 0);
     for (size_t b = 0; b < h.desc.size(); ++b) {
         const int e0 = h.desc[b].z, ne = h.desc[b].w;
+        (narrow && ne <= h.cap ? h.nnz16 : h.nnz32) += ne;
         if (ne > h.cap) continue;
         std::copy(val.begin() + e0, val.begin() + e0 + ne, h.val.begin() + b * h.cap);
         for (int k = 0; k < ne; ++k) {

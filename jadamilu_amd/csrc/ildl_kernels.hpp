@@ -109,6 +109,7 @@ struct StreamHost {
     std::vector<int> cbase, c32;
     std::vector<unsigned short> off, c16;
     std::vector<T> val;
+    long nnz16 = 0, nnz32 = 0;  // entries (no padding) by the column width they are read with
 };
 template <typename T>
 StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx,

@@ -26,7 +26,8 @@ def _hub(n, k):
 
 
 def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=300):
-    """The apply against the oracle's; the kernel forms chosen."""
+    """The apply against the oracle's; the factor, the kernel forms chosen and
+    the bytes that a forward sweep of the first level is said to take."""
     from jadamilu_amd.ildl import IldlFactor
     from jadamilu_amd.jd import Context
     if not torch.cuda.is_available():
@@ -52,9 +53,35 @@ def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=3
         zo = O.ildl_apply(ex, r, sweeps=sweeps)
         tol = 2e-5 if single else 1e-12
         assert np.linalg.norm(zd.cpu().numpy() - zo) <= tol * np.linalg.norm(zo)
-    forms = ctx.ildl_level_forms()
+    forms, nbytes = ctx.ildl_level_forms(), ctx.ildl_time_sweep(1)[1]
     ctx.close()
-    return forms
+    return ex, forms, nbytes
+
+
+def _stream_bytes(level, single):
+    """What a forward sweep in the CSR-stream form reads and writes when the
+    factor's own order is kept, and its entries by the width of their columns:
+    blocks of up to 256 rows and 512 entries (1024 from 800,000 on); 16-bit
+    columns if all blocks span less than 65,536 of them."""
+    ptr, idx = level["lb_ptr"].astype(np.int64), level["lb_idx"]
+    n, nnz = ptr.size - 1, int(ptr[-1])
+    cap = 1024 if nnz >= 800000 else 512
+    assert np.diff(ptr).max() <= cap
+    r, nblk, narrow, wide = 0, 0, 0, 0
+    while r < n:
+        r0 = r
+        r = min(n, r0 + 256, int(np.searchsorted(ptr, ptr[r0] + cap, "right")) - 1)
+        cols = idx[ptr[r0]:ptr[r]]
+        nblk += 1
+        if cols.size and int(cols.max()) - int(cols.min()) >= 65536:
+            wide += cols.size
+        else:
+            narrow += cols.size
+    if wide:
+        narrow, wide = 0, wide + narrow
+    size = 4 if single else 8
+    total = (size * nnz + 2 * narrow + 4 * wide + 2 * (n + nblk) + 20 * nblk + 3 * size * n)
+    return total, narrow, wide
 
 
 # rows around the 512 entries that a block of the small CSR-stream form holds
@@ -70,7 +97,7 @@ def test_stream_rows_at_the_block_size(k, single):
 @pytest.mark.parametrize("k,form", [(100, [8, 8]), (129, [8, 8]), (130, [1, 8]),
                                     (4000, [8, 8, 1])])
 def test_long_row_among_short_ones(k, form):
-    forms = _check(lambda: _hub(4000, k), {}, 3, dense_max=0)
+    _, forms, _ = _check(lambda: _hub(4000, k), {}, 3, dense_max=0)
     assert forms[0][:len(form)] == form
 
 
@@ -89,9 +116,38 @@ def test_fused_ends_of_the_sweeps(gen, spd, sweeps, form, coupling, graph):
                single=single, spd=spd, dense_max=50)
 
 
+# the column widths of the CSR-stream form, 16 bits and 32 bits at both block
+# sizes; the bytes that the sweep reports say which was taken
+@pytest.mark.parametrize("gen,widths", [
+    (lambda: M.laplace((30, 29, 28)), (True, False)),
+    (lambda: M.laplace((300, 290)), (False, True)),
+    (lambda: M.laplace((62, 61, 60)), (False, True)),
+])
+@pytest.mark.parametrize("single", [False, True])
+def test_stream_column_widths(gen, widths, single):
+    ex, _, nbytes = _check(gen, {"ildl_form": 1, "ildl_storage": 0}, 2, single=single)
+    total, narrow, wide = _stream_bytes(ex["levels"][0], single)
+    assert (narrow > 0, wide > 0) == widths
+    assert nbytes == total
+
+
 # a level large enough for the blocks of 1024 entries
 def test_stream_wide_blocks():
     _check(lambda: M.laplace((64, 63, 61)), {"ildl_form": 1}, 2)
+
+
+def test_stream_long_row_among_wide_blocks():
+    """A coupling block of more than 800,000 entries, so in blocks of 1024, with
+    a row of some thousand entries."""
+    def gen():
+        parts = [M.laplace((86, 85, 84)), _hub(30000, 30000)]
+        n = parts[0][0].size - 1
+        return (np.concatenate([parts[0][0][:-1], parts[1][0] + parts[0][0][-1] - 1]),
+                np.concatenate([parts[0][1], parts[1][1] + n]),
+                np.concatenate([p[2] for p in parts]))
+    ex, _, _ = _check(gen, {"ildl_form": 1}, 2)
+    ptr = ex["levels"][0]["lc_ptr"]
+    assert ptr[-1] >= 800000 and np.diff(ptr).max() > 1024
 
 
 def test_apply_on_a_stream_under_capture():
