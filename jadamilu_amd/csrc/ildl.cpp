@@ -625,7 +625,7 @@ class IldlImpl : public IldlImplBase {
         v.cbase = track(dev_upload(ctx_->stream, h.cbase));
         v.off = track(dev_upload(ctx_->stream, h.off));
         if (!h.c16.empty()) v.c16 = track(dev_upload(ctx_->stream, h.c16));
-        else v.c32 = track(dev_upload(ctx_->stream, h.c32));
+        if (!h.c32.empty()) v.c32 = track(dev_upload(ctx_->stream, h.c32));
         v.val = track(dev_upload(ctx_->stream, h.val));
         d.nnz16 = h.nnz16;
         d.nnz32 = h.nnz32;

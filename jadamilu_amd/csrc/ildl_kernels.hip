@@ -238,7 +238,16 @@ __global__ __launch_bounds__(kB) void k_stream(StreamView<T> M, const int *__res
         v[u] = ((const T2 *)M.val)[k];
     }
     const int4 d = M.desc[blk];
-    const int cb = NARROW ? M.cbase[blk] : 0;
+    int cb = NARROW ? M.cbase[blk] : 0;
+    if (NARROW && cb < 0) {  // a wide block
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            const int2 q = ((const int2 *)M.c32)[(long)~cb * (CAP / 2) + tid + u * kB];
+            c0[u] = q.x;
+            c1[u] = q.y;
+        }
+        cb = 0;
+    }
     const int r0 = d.x, nr = d.y, e0 = d.z, ne = d.w;
     if (ne > CAP) {  // one long row
         double s0 = 0.0, s1 = 0.0;
@@ -407,13 +416,21 @@ void ildl_stream(const Put &s, const StreamView<T> &M, const int *idx, const T *
 // 609k 5.4 / 5.8, 988k 6.3 / 6.0, 1.2M 5.8 / 5.4, 7.5M 28.7 / 24.7.
 static constexpr long kStreamWide = 800000;
 
+// Columns take 16 bits where at most one block in this many is wide (spans
+// 65,536 columns or more): a wide block loads its columns again, in 32 bits, once
+// it knows its descriptor.  100^3 Laplacian, 17 wide blocks of 3,623: sweep 14.7
+// -> 14.1 us, apply 569 -> 560 us, with FP32 values 11.6 -> 10.5 and 453 -> 434.
+// With a quarter to a third of wide blocks (Anderson L = 48 and 60) there is no
+// difference.
+static constexpr size_t kFewWide = 4;
+
 template <typename T>
 StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx,
                            const std::vector<T> &val) {
     StreamHost<T> h;
     const int nnz = ptr[nrows];
     h.cap = nnz >= kStreamWide ? 1024 : 512;
-    bool narrow = true;
+    int wide = 0;
     int r = 0;
     while (r < nrows) {
         const int r0 = r, e0 = ptr[r];
@@ -427,26 +444,28 @@ StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::ve
                 cmax = std::max(cmax, idx[k]);
             }
         if (cmin > cmax) cmin = cmax = 0;
-        narrow = narrow && (long)cmax - cmin < 65536;
         h.desc.push_back(make_int4(r0, r - r0, e0, ne));
-        h.cbase.push_back(cmin);
+        h.cbase.push_back((long)cmax - cmin < 65536 ? cmin : ~wide++);
         // entry range of each row, from the block's first entry (a long row's
         // range is not read)
         for (int i = r0; i <= r; ++i) h.off.push_back((unsigned short)(ptr[i] - e0));
     }
     const size_t slots = h.desc.size() * h.cap;
+    const bool narrow = wide * kFewWide <= h.desc.size();
     h.val.assign(slots, T(0));
     if (narrow) h.c16.assign(slots, 0);
-    else h.c32.assign(slots, 0);
+    h.c32.assign(narrow ? (size_t)wide * h.cap : slots, 0);
     for (size_t b = 0; b < h.desc.size(); ++b) {
-        const int e0 = h.desc[b].z, ne = h.desc[b].w;
-        (narrow && ne <= h.cap ? h.nnz16 : h.nnz32) += ne;
+        const int e0 = h.desc[b].z, ne = h.desc[b].w, cb = h.cbase[b];
+        const bool n16 = narrow && cb >= 0 && ne <= h.cap;
+        (n16 ? h.nnz16 : h.nnz32) += ne;
         if (ne > h.cap) continue;
         std::copy(val.begin() + e0, val.begin() + e0 + ne, h.val.begin() + b * h.cap);
-        for (int k = 0; k < ne; ++k) {
-            if (narrow) h.c16[b * h.cap + k] = (unsigned short)(idx[e0 + k] - h.cbase[b]);
-            else h.c32[b * h.cap + k] = idx[e0 + k];
-        }
+        if (n16)
+            for (int k = 0; k < ne; ++k) h.c16[b * h.cap + k] = (unsigned short)(idx[e0 + k] - cb);
+        else
+            std::copy(idx.begin() + e0, idx.begin() + e0 + ne,
+                      h.c32.begin() + (narrow ? (size_t)~cb : b) * h.cap);
     }
     return h;
 }

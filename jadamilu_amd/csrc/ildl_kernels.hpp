@@ -87,8 +87,9 @@ void ildl_csr(const Put &s, int lpr, int nrows, const int *ptr, const int *idx, 
 // rows) each, or one longer row, streamed through LDS with coalesced loads.
 // Block b's entries are laid out again from entry b*cap on (padded with zeros),
 // so that a block finds them without looking anything up: values val, and
-// columns c16 (offsets from cbase[b]) if every block's span less than 2^16, else
-// c32.  desc[b] = {first row, rows, first entry in the CSR, entries} (a longer
+// columns c16 (offsets from cbase[b] >= 0) if most blocks' span less than 2^16,
+// else c32.  Beside c16, c32 holds only the blocks whose columns span more, block
+// b from entry ~cbase[b]*cap on.  desc[b] = {first row, rows, first entry in the CSR, entries} (a longer
 // row is read from there); off[row + b] and the next are a row's entry range
 // from the block's first entry.
 template <typename T>
@@ -98,7 +99,7 @@ struct StreamView {
     const int4 *desc = nullptr;
     const int *cbase = nullptr;
     const unsigned short *off = nullptr;
-    const unsigned short *c16 = nullptr;  // or
+    const unsigned short *c16 = nullptr;
     const int *c32 = nullptr;
     const T *val = nullptr;
 };

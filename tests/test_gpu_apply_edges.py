@@ -58,16 +58,17 @@ def _check(gen, options, sweeps, coupling=0, single=False, spd=True, dense_max=3
     return ex, forms, nbytes
 
 
-def _stream_bytes(level, single):
+def _stream_bytes(level, value, vector):
     """What a forward sweep in the CSR-stream form reads and writes when the
     factor's own order is kept, and its entries by the width of their columns:
     blocks of up to 256 rows and 512 entries (1024 from 800,000 on); 16-bit
-    columns if all blocks span less than 65,536 of them."""
+    columns where a block spans less than 65,536 of them, if three quarters of
+    the blocks do.  value, vector: bytes of an entry and of a vector's."""
     ptr, idx = level["lb_ptr"].astype(np.int64), level["lb_idx"]
     n, nnz = ptr.size - 1, int(ptr[-1])
     cap = 1024 if nnz >= 800000 else 512
     assert np.diff(ptr).max() <= cap
-    r, nblk, narrow, wide = 0, 0, 0, 0
+    r, nblk, wide_blocks, narrow, wide = 0, 0, 0, 0, 0
     while r < n:
         r0 = r
         r = min(n, r0 + 256, int(np.searchsorted(ptr, ptr[r0] + cap, "right")) - 1)
@@ -75,12 +76,12 @@ def _stream_bytes(level, single):
         nblk += 1
         if cols.size and int(cols.max()) - int(cols.min()) >= 65536:
             wide += cols.size
+            wide_blocks += 1
         else:
             narrow += cols.size
-    if wide:
+    if 4 * wide_blocks > nblk:
         narrow, wide = 0, wide + narrow
-    size = 4 if single else 8
-    total = (size * nnz + 2 * narrow + 4 * wide + 2 * (n + nblk) + 20 * nblk + 3 * size * n)
+    total = value * nnz + 2 * narrow + 4 * wide + 2 * (n + nblk) + 20 * nblk + 3 * vector * n
     return total, narrow, wide
 
 
@@ -116,17 +117,21 @@ def test_fused_ends_of_the_sweeps(gen, spd, sweeps, form, coupling, graph):
                single=single, spd=spd, dense_max=50)
 
 
-# the column widths of the CSR-stream form, 16 bits and 32 bits at both block
-# sizes; the bytes that the sweep reports say which was taken
-@pytest.mark.parametrize("gen,widths", [
-    (lambda: M.laplace((30, 29, 28)), (True, False)),
-    (lambda: M.laplace((300, 290)), (False, True)),
-    (lambda: M.laplace((62, 61, 60)), (False, True)),
+# the column widths of the CSR-stream form, 16 bits, some blocks in 32 and all in
+# 32, at both block sizes; the bytes that the sweep reports say which was taken
+@pytest.mark.parametrize("gen,spd,widths", [
+    (lambda: M.laplace((30, 29, 28)), True, (True, False)),
+    (lambda: M.laplace((46, 45, 44)), True, (True, True)),
+    (lambda: M.laplace((48, 46, 44)), True, (False, True)),
+    (lambda: M.anderson(42, 16.5, 1), False, (True, False)),
+    (lambda: M.anderson(44, 16.5, 1), False, (True, True)),
+    (lambda: M.laplace((62, 61, 60)), True, (False, True)),
 ])
 @pytest.mark.parametrize("single", [False, True])
-def test_stream_column_widths(gen, widths, single):
-    ex, _, nbytes = _check(gen, {"ildl_form": 1, "ildl_storage": 0}, 2, single=single)
-    total, narrow, wide = _stream_bytes(ex["levels"][0], single)
+def test_stream_column_widths(gen, spd, widths, single):
+    ex, _, nbytes = _check(gen, {"ildl_form": 1, "ildl_storage": 0}, 2, single=single, spd=spd)
+    total, narrow, wide = _stream_bytes(ex["levels"][0], 4 if single else 8,
+                                        4 if single and spd else 8)
     assert (narrow > 0, wide > 0) == widths
     assert nbytes == total
 
