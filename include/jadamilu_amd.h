@@ -367,8 +367,8 @@ int jdhip_tall_gemm(jdhip_ctx *ctx, long n, int k, int j, const double *v_dev, l
  * the default; 1 = every interval reads 0 s, so the reference's floors
  * decide, as on a machine where the problem is small: the set-up sequence and
  * the suggested DROPTOL then follow from the residual history alone).
- * 0 on success, -2 for an
- * unknown name, -3 for an invalid value. */
+ * 0 on success, -2 for an unknown name, -3 for an invalid value, -4 for an error
+ * of the device where an option takes effect at once (jdhip_last_error). */
 int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value);
 
 /* z = P^-1 r with the preconditioner currently held by ctx (diagonal or

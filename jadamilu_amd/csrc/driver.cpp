@@ -1260,9 +1260,7 @@ int jdhip_reset(jdhip_ctx *ctx) {
     return 0;
 }
 
-int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value) {
-    if (!ctx || !name) return -1;
-    Solver &S = *ctx->S;
+static int set_option(Solver &S, const char *name, double value) {
     std::string k(name);
     if (k == "ildl_sweeps") S.ildl_sweeps = (int)value;
     else if (k == "ildl_ordering") S.ildl_ordering = (int)value;
@@ -1299,10 +1297,23 @@ int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value) {
     }
     else if (k == "ildl_graph") {
         S.ildl_graph = (int)value;
-        if (S.ildl && S.ildl->ready()) S.ildl->impl()->set_graphs(S.ildl_graph);
+        if (S.ildl && S.ildl->ready()) {
+            JDHIP_CHECK(hipSetDevice(S.ctx.device));
+            S.ildl->impl()->set_graphs(S.ildl_graph);
+        }
     }
     else return -2;
     return 0;
+}
+
+int jdhip_set_option(jdhip_ctx *ctx, const char *name, double value) {
+    if (!ctx || !name) return -1;
+    try {
+        return set_option(*ctx->S, name, value);
+    } catch (const std::exception &e) {
+        set_err(ctx, e.what());
+        return -4;
+    }
 }
 
 int jdhip_spmm(jdhip_ctx *ctx, int k, const double *x_dev, long ldx, double *y_dev, long ldy) {

@@ -354,6 +354,8 @@ class Context:
 
     def set_option(self, name, value):
         rc = self._L.jdhip_set_option(self.h, name.encode(), float(value))
+        if rc == -4:
+            raise RuntimeError(self.error())
         if rc != 0:
             raise ValueError(f"unknown option {name}")
 
