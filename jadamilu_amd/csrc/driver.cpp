@@ -181,6 +181,7 @@ struct Solver {
     bool build_dia(CsrDev &M, int n_, const int *ia_, const int *ja_, const double *a_);
     void build_sell(CsrDev &M, int n_, const std::vector<int> &rp, const std::vector<int> &col,
                     const std::vector<double> &val);
+    void ensure_sell(CsrDev &M);
     double A_fp = 0.0;
     static double fingerprint(int n_, const int *ia_, const int *ja_, const double *a_) {
         double s = (double)n_ + 1e-3 * (double)ia_[n_];
@@ -385,6 +386,23 @@ void Solver::build_sell(CsrDev &A, int n_, const std::vector<int> &rp,
     A.nslices = ns;
     A.s_entries = ent;
     A.s_idx_bytes = iptr[ns];
+}
+
+// The sliced-ELL copy of a matrix in the diagonal form, which has none until it
+// is asked for.
+void Solver::ensure_sell(CsrDev &M) {
+    if (M.nslices > 0 || M.dia.nd == 0) return;
+    JDHIP_CHECK(hipSetDevice(ctx.device));
+    std::vector<int> rp(M.n + 1), col(M.nnz);
+    std::vector<double> val(M.nnz);
+    auto fetch = [&](void *dst, const void *src, size_t bytes) {
+        JDHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx.stream));
+    };
+    fetch(rp.data(), M.rowptr, sizeof(int) * rp.size());
+    fetch(col.data(), M.col, sizeof(int) * col.size());
+    fetch(val.data(), M.val, sizeof(double) * val.size());
+    JDHIP_CHECK(hipStreamSynchronize(ctx.stream));
+    build_sell(M, M.n, rp, col, val);
 }
 
 // Pick lanes-per-row by timing the candidates on this matrix.
@@ -1271,7 +1289,7 @@ static int set_option(Solver &S, const char *name, double value) {
     else if (k == "ildl_dense_max") S.ildl_dense_max = (int)value;
     else if (k == "spmv_lanes") {
         S.A.lpr = (int)value;
-        if (S.A.lpr == 0 && S.A.nslices == 0 && S.A.dia.nd > 0) S.A.lpr = jdhip::kLprDia;
+        if (S.A.lpr == 0) S.ensure_sell(S.A);
     }
     else if (k == "inner_fp32") S.inner_fp32 = value != 0.0;
     else if (k == "inner_spmv64") S.inner_spmv64 = value != 0.0;

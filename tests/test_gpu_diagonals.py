@@ -153,3 +153,29 @@ def test_fp32_inner_solver_on_diagonals(spmv64):
     assert r.info == 0 and r.stats["spmv_lanes"] == -2
     np.testing.assert_allclose(r.eigs, lam, rtol=1e-10)
     ctx.close()
+
+
+def test_other_formats_of_a_matrix_on_diagonals():
+    """Option spmv_lanes selects every format on a matrix that took the diagonal
+    form, the sliced ELL included, and back."""
+    from jadamilu_amd.jd import Context
+    _dev()
+    n = 67 * 63
+    X = torch.randn(2, n, dtype=torch.float64, device="cuda:0")
+    ctx = Context(0)
+    ctx.set_matrix(*M.laplace((67, 63)))
+    results = []
+    for lanes in (-2, 0, 4, -2):
+        ctx.set_option("spmv_lanes", lanes)
+        assert ctx.stats()["spmv_lanes"] == lanes
+        Y = torch.zeros(3, n, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ctx.spmv(X.data_ptr(), Y[0].data_ptr())
+        ctx.spmm(2, X.data_ptr(), n, Y[1].data_ptr(), n)
+        torch.cuda.synchronize()
+        results.append(Y)
+    ctx.close()
+    # five terms a row, of absolute sum 8 max|x| at most, in different orders
+    bound = 2 * 6 * 2.0 ** -53 * 8 * float(X.abs().max())
+    for Y in results[1:]:
+        assert float((Y - results[0]).abs().max()) <= bound
