@@ -1,9 +1,9 @@
 """The diagonal form of the symmetric products against the CSR form of the same
 matrix, and the matrices that must not take it.
 
-Both forms add a row's few products in double in another order: the results
-agree to a few units of the row's largest term (1e-15 of the sum of absolute
-terms is taken, twice the worst case of seven terms being 7 * 2^-53 * 2).
+Both forms add a row's m products in double in another order: each is off by
+m * 2^-53 of the sum of absolute terms at most, so they agree to twice that (one
+more for the rounding of that sum itself).
 """
 import numpy as np
 import pytest
@@ -108,7 +108,9 @@ def test_diagonal_form_equals_csr(gen, diagonal, k):
     z, _ = _products(mat, X, 8)
     assert (form == -2) == diagonal
     scale, _ = _products((mat[0], mat[1], np.abs(mat[2])), X.abs(), 8)
-    assert (np.abs(y - z) <= 1e-15 * scale).all()
+    rows, cols = np.repeat(np.arange(n), np.diff(mat[0])), mat[1] - 1
+    m = np.bincount(rows, minlength=n) + np.bincount(cols[rows != cols], minlength=n)
+    assert (np.abs(y - z) <= 2 * (m + 1) * 2.0 ** -53 * scale).all()
 
 
 def test_infinities_stay_where_the_matrix_puts_them():
