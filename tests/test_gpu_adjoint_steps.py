@@ -39,7 +39,7 @@ def _check(rows, n, k, rng):
 
 
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 12, 13, 16, 17, 33, 64])
-@pytest.mark.parametrize("n", [1, 63, 65, 1500])
+@pytest.mark.parametrize("n", [1, 63, 65, 1500, 32767, 32768 + 65])
 def test_gradients_at_every_step(n, k):
     if not torch.cuda.is_available():
         pytest.skip("no HIP device")
@@ -50,10 +50,10 @@ def test_gradients_at_every_step(n, k):
     _check(rows, n, k, rng)
 
 
-# Row lengths of three waves of 64 rows and a partial one, at the limits up to
-# which a wave gives each lane a row (16 entries a row, 512 in its 64 rows): all
-# at a limit, one entry over it, a long row among short ones, and waves that
-# decide differently side by side.
+# Row lengths of 64 rows at the limits up to which a wave gives each lane a row (16
+# entries a row, 512 in its 64 rows): all at a limit, one entry over it, a long
+# row among short ones; beside waves that decide otherwise and as a last wave of
+# few rows.  Matrices of at least 32,768 rows have such waves.
 LENGTHS = {
     "row 16": [16] + [0] * 63, "row 17": [17] + [0] * 63,
     "wave 512": [8] * 64, "wave 513": [8] * 63 + [9],
@@ -68,8 +68,9 @@ LENGTHS = {
 def test_gradients_at_the_limits_of_a_wave(name, tail, k):
     if not torch.cuda.is_available():
         pytest.skip("no HIP device")
-    lengths = [5] * 64 + LENGTHS[name] + [12] * 64 + LENGTHS[name][-tail:]
+    lengths = [1] * 32768 + [5] * 64 + LENGTHS[name] + [12] * 64 + LENGTHS[name][-tail:]
     n = len(lengths)
     rng = np.random.default_rng(k)
     # (any columns: the kernel does not ask for the upper triangle)
-    _check([np.sort(rng.choice(n, m, replace=False)) for m in lengths], n, k, rng)
+    _check([np.array([i]) if i < 32768 else np.sort(rng.choice(n, m, replace=False))
+            for i, m in enumerate(lengths)], n, k, rng)
