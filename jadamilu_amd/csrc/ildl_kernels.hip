@@ -420,9 +420,9 @@ static constexpr long kStreamWide = 800000;
 // 65,536 columns or more): a wide block loads its columns again, in 32 bits, once
 // it knows its descriptor.  100^3 Laplacian, 17 wide blocks of 3,623: sweep 14.7
 // -> 14.1 us, apply 569 -> 560 us, with FP32 values 11.6 -> 10.5 and 453 -> 434.
-// With a quarter to a third of wide blocks (Anderson L = 48 and 60) there is no
-// difference.
-static constexpr size_t kFewWide = 4;
+// With a quarter of wide blocks it is no gain: Anderson L = 100, level 2 (10.2M
+// entries), 34.1 and 33.3 us all in 32 bits, 34.2 and 34.0 in both widths.
+static constexpr size_t kFewWide = 8;
 
 template <typename T>
 StreamHost<T> build_stream(int nrows, const std::vector<int> &ptr, const std::vector<int> &idx,

@@ -62,7 +62,7 @@ def _stream_bytes(level, value, vector):
     """What a forward sweep in the CSR-stream form reads and writes when the
     factor's own order is kept, and its entries by the width of their columns:
     blocks of up to 256 rows and 512 entries (1024 from 800,000 on); 16-bit
-    columns where a block spans less than 65,536 of them, if three quarters of
+    columns where a block spans less than 65,536 of them, if seven eighths of
     the blocks do.  value, vector: bytes of an entry and of a vector's."""
     ptr, idx = level["lb_ptr"].astype(np.int64), level["lb_idx"]
     n, nnz = ptr.size - 1, int(ptr[-1])
@@ -79,7 +79,7 @@ def _stream_bytes(level, value, vector):
             wide_blocks += 1
         else:
             narrow += cols.size
-    if 4 * wide_blocks > nblk:
+    if 8 * wide_blocks > nblk:
         narrow, wide = 0, wide + narrow
     total = value * nnz + 2 * narrow + 4 * wide + 2 * (n + nblk) + 20 * nblk + 3 * vector * n
     return total, narrow, wide
