@@ -20,8 +20,8 @@
 // Cache does not hold them): 128^3 Laplacian 35.9 -> 22.1 us (107 MB of HBM
 // traffic instead of 182 MB), and with two in turn 35.0 -> 14.5 us; Anderson
 // L = 100 with two in turn 11.6 -> 8.3 us; ten vectors of it 79.2 -> 72.7 us
-// (260 MB at 3.7 TB/s: bound by the vectors' streams, of which a wave has more
-// than it can keep full).
+// (239 MB of HBM traffic for 192 MB needed, and 26.8 million L1 accesses, 44 us
+// of the L1's time: neither alone is the whole).
 #include "kernels.hpp"
 #include "reduce.hpp"
 #include "xcd.hpp"
